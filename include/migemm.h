@@ -372,7 +372,8 @@ int migemm_set_gemm_policy(int policy, int *previous);
                                       or MIGEMM_TILE_128x256 */
 #define MIGEMM_TUNE_SPLITK 2       /* tiled kernel's k ranges: S in 1..64 */
 #define MIGEMM_TUNE_DIRECT 3       /* operands loaded straight into LDS: 1 never,
-                                      2 wherever the kernel applies (also split 128x256) */
+                                      2 wherever the kernel applies (also split 128x256);
+                                      either value keeps every product on the fp32 MFMA */
 #define MIGEMM_TUNE_SMALL_TILES 4  /* small-output kernel's 32x32 tiles: 1 never,
                                       2 always (M, N > 16) */
 #define MIGEMM_TUNE_SMALL_SPLITK 5 /* small-output kernel's k ranges: S in 1..64 */
@@ -381,7 +382,10 @@ int migemm_set_tuning(int key, int value, int *previous);
 
 /* Writes a one-line description of the kernel the last GEMM / permute / column-sum call of
  * this host thread ran (family, output tile, k ranges, load width, shape, layout) into
- * buf (NUL-terminated, truncated to len). For tests and tuning; the reference has none. */
+ * buf (NUL-terminated, truncated to len). For tests and tuning; the reference has none.
+ * A large product of the tiled family that runs on the bf16 matrix cores (under the AUTO
+ * policy, with no tiled tuning override) is described by the fp32 plan it replaces; its own
+ * tile and k ranges follow from that plan and the sizes. */
 int migemm_last_plan(char *buf, size_t len);
 
 /* (5) Measurement. Streams src[0 .. n) once -- `blocks` work-groups, each a contiguous

@@ -360,7 +360,7 @@ static int run_gemm(hipStream_t stream, const GemmDesc &desc) {
     if (tiny_preferred(d)) return launch_gemm_tiny(stream, d);
     if (panel_preferred(d)) return launch_gemm_panel(stream, d);
     if (small_preferred(d)) return launch_gemm_small(stream, d);
-    return launch_gemm_tiled(stream, d);
+    return launch_gemm_tiled(stream, d, policy == MIGEMM_POLICY_AUTO);
 }
 
 // C = opA(A) opB(B) + opA(A2) opB(B2) (+ bias) for a descriptor with a second operand pair:

@@ -551,7 +551,7 @@ constexpr double kUnalignedRate64 = 0.85, kUnalignedRate128 = 0.95;
 constexpr double kPartialBytesPerUs = 6e6;
 }  // namespace
 
-int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d) {
+int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d, bool automatic) {
     // Operand orientation: A is K-contiguous unless transposed; B is K-contiguous only
     // when transposed.
     const bool akc = !d.transA;
@@ -821,6 +821,23 @@ int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d) {
             big = best == c2 ? 2 : (best == c1 ? 1 : 0);
         }
     }
+    // Operands split into bf16 parts on the bf16 matrix cores (gemm_split.hip), where their
+    // estimate is below 0.95 of this plan's.
+    SplitPlan split_plan = {0, 0, 1, 0.0};
+    if (automatic && fits && direct_mode == 0 && tuning(MIGEMM_TUNE_TILE) == 0 &&
+        tuning(MIGEMM_TUNE_SPLITK) == 0 && cfg != 32 && d.K >= 128) {
+        const TileShape shape = cfg == 64 ? T64 : big == 0 ? T128 : big == 1 ? T128x256 : T256;
+        const int bm = big == 2 ? 256 : cfg, bn = big >= 1 ? 256 : cfg;
+        // rates of operands loaded 4 bytes per lane as in the k-range estimates above
+        const double e = direct ? 1.0 : cfg == 64 ? kUnalignedRate64 : kUnalignedRate128;
+        const double t_plan =
+            est(tiles(bm, bn) * splits, (double)bm * bn, (double)d.K / splits,
+                kDirectFit[shape], e) +
+            (splits > 1 ? (2.0 * splits + 1) * d.M * d.N * 4.0 * d.batch / kPartialBytesPerUs
+                        : 0.0);
+        const SplitPlan best = plan_split(d, splits);
+        if (best.us < 0.95 * t_plan) split_plan = best;
+    }
     // tuning overrides (migemm_set_tuning), validated when they were set
     const int force_tile = tuning(MIGEMM_TUNE_TILE);
     const int force_split = tuning(MIGEMM_TUNE_SPLITK);
@@ -857,6 +874,31 @@ int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d) {
         a.partial =
             partial_buffer(stream, d, (size_t)splits * d.batch * d.M * d.N * sizeof(float), &st);
         if (a.partial == nullptr) return st;
+    }
+    if (split_plan.bm != 0 && split_plan.splits > splits) {
+        // more k ranges than the plan's: where their partial sums are not to be had (a
+        // stream being captured without a workspace), the plan runs as it is
+        int st = MIGEMM_OK;
+        a.partial = partial_buffer(
+            stream, d, (size_t)split_plan.splits * d.batch * d.M * d.N * sizeof(float), &st);
+        if (a.partial == nullptr) {
+            clear_error();
+            split_plan.bm = 0;
+        }
+    }
+    if (split_plan.bm != 0) {
+        TiledArgs sa = a;
+        sa.write_back = !rows64;
+        const int rc = launch_gemm_split(stream, sa, split_plan, akc, bkc);
+        // the record keeps the decomposition it replaces, whose non-empty ranges are
+        const int nk = cfg == 128 && big == 0 ? (d.K + 15) / 16 : nk32;
+        const int per = (nk + std::min(splits, nk) - 1) / std::min(splits, nk);
+        record_plan("tiled-direct", d, cfg == 128 && big == 2 ? 256 : cfg,
+                    cfg == 128 && big >= 1 ? 256 : cfg, (nk + per - 1) / per,
+                    wa == 4 && wb == 4 ? 16 : 4);
+        if (rc != MIGEMM_OK || sa.splits == 1) return rc;
+        return launch_reduce_slices(stream, sa.partial, sa.splits, d.batch, d.M, d.N, d.bias,
+                                    d.C, d.ldc, d.sC, d.accumulate);
     }
     int rc;
     switch (cfg) {

@@ -110,7 +110,9 @@ bool plan_only();
 int launch_status(const char *what);
 
 // Launchers. They assume a validated descriptor and only enqueue work.
-int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d);
+// automatic: the dispatcher's own choice (not a forced family), which may run the product on
+// the bf16 matrix cores (gemm_split.hip).
+int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d, bool automatic = false);
 int launch_gemm_skinny(hipStream_t stream, const GemmDesc &d);
 // M <= 4 (gemm_skinny_kernel for B not transposed, gemv_rows_kernel for B transposed).
 bool skinny_supported(const GemmDesc &d);

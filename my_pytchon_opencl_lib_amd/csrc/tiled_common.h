@@ -164,4 +164,16 @@ __device__ __forceinline__ void store_tile(const TiledArgs &p, const TileCoord &
 int launch_gemm_direct(hipStream_t stream, TiledArgs &a, int bm, int bn, bool akc, bool bkc,
                        int wa = 4, int wb = 4);
 
+// Tiles of bm x bn computed on the bf16 matrix cores from operands split into three bf16
+// parts (gemm_split.hip). plan_split: the tile shape and k ranges with the least estimated
+// time, when the fp32 plan has plan_splits ranges; launch_gemm_split runs them (on return
+// `a` holds the grid and the non-empty range count).
+struct SplitPlan {
+    int bm, bn, splits;
+    double us;
+};
+SplitPlan plan_split(const GemmDesc &d, int plan_splits);
+int launch_gemm_split(hipStream_t stream, TiledArgs &a, const SplitPlan &plan, bool akc,
+                      bool bkc);
+
 }  // namespace migemm

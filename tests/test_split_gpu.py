@@ -1,0 +1,164 @@
+"""GPU tests of gemm_split_kernel: large products on the bf16 matrix cores, every operand
+value split into three bf16 parts (gemm_split.hip), taken by the dispatcher's own choice.
+
+The shapes reach its three tiles (256x256, 256x128, 128x128), ragged M and N, k-tiles of 16
+with every kind of tail, and k ranges. Small-integer operands make the exact answer known in
+any summation order. On random operands the error against fp64 is compared with that of the
+fp32 kernels on the same call (direct loads forced: no split), which it must not exceed, and
+the bits must differ, which shows that the split kernel ran."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from my_pytchon_opencl_lib_amd import _native
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(0, 0), (0, 1), (1, 0), (1, 1)]
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def run(ta, tb, M, N, K, a, lda, sA, b, ldb, sB, bias, c, ldc, sC, batch=1, acc=False):
+    _native.call("migemm_gemm_strided_batched_ex",
+                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), ta, tb, M, N, K,
+                 ctypes.c_void_p(a.data_ptr()), lda, sA, ctypes.c_void_p(b.data_ptr()), ldb, sB,
+                 None if bias is None else ctypes.c_void_p(bias.data_ptr()),
+                 ctypes.c_void_p(c.data_ptr()), ldc, sC, batch, int(acc))
+
+
+def case(M, K, N, ta, tb, batch=1, pad=0, off=0, ints=True, seed=0):
+    """Operands as (device buffer view, ld, stride) and their fp64 op(A), op(B): rows padded
+    by `pad` NaN, the first element `off` floats into the buffer."""
+    g = torch.Generator(device="cuda:0").manual_seed(seed)
+
+    def one(rows, cols):
+        ld = cols + pad
+        buf = torch.full((off + batch * rows * ld,), float("nan"), device="cuda:0")
+        x = (torch.randint(-4, 5, (batch, rows, cols), generator=g, device="cuda:0").float()
+             if ints else torch.randn(batch, rows, cols, generator=g, device="cuda:0"))
+        buf[off:].view(batch, rows, ld)[:, :, :cols] = x
+        return buf[off:], ld, rows * ld, x.double()
+
+    a, lda, sA, a64 = one(*((K, M) if ta else (M, K)))
+    b, ldb, sB, b64 = one(*((N, K) if tb else (K, N)))
+    a64 = a64.transpose(1, 2).contiguous() if ta else a64
+    b64 = b64.transpose(1, 2).contiguous() if tb else b64
+    return (a, lda, sA), (b, ldb, sB), a64, b64
+
+
+# 128x128 (2100 x 1009 x 1300), 256x128 and 256x256 tiles; K % 16 = 0, 1, 15 and 9
+SHAPES = [(2100, 1009, 1300), (4097, 144, 3073), (5000, 511, 2049), (3073, 2048, 4225)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+def test_split_exact(M, K, N, ta, tb):
+    """Odd sizes, rows off 16-byte boundaries, NaN between the rows; bias and C += result."""
+    for pad, off, bias, acc in [(0, 0, False, False), (3, 1, True, True)]:
+        say("split exact", M, K, N, ta, tb, pad, off, bias, acc)
+        (a, lda, sA), (b, ldb, sB), a64, b64 = case(M, K, N, ta, tb, pad=pad, off=off, seed=K)
+        bv = torch.arange(N, device="cuda:0").remainder(41).sub(20).float() if bias else None
+        c = torch.full((M, N + pad), 7.0 if acc else float("nan"), device="cuda:0")
+        run(ta, tb, M, N, K, a, lda, sA, b, ldb, sB, bv, c, N + pad, 0, acc=acc)
+        expect = (a64 @ b64)[0]
+        if bias:
+            expect = expect + bv.double()
+        if acc:
+            expect = expect + 7.0
+        assert torch.equal(c[:, :N], expect.float())
+        if pad:
+            assert bool((c[:, N:] == 7.0).all() if acc else c[:, N:].isnan().all())
+
+
+# (M, K, N, batch): one range; k ranges as the fp32 plan has them (6400 x 4096 x 512 in 3,
+# 500 x 12000 x 6565 in 6); more ranges than it has (512 x 6400 x 4096); a batch
+RANDOM = [(2100, 1009, 1300, 1), (4096, 512, 3000, 1), (4096, 2048, 4096, 1),
+          (6400, 4096, 512, 1), (500, 12000, 6565, 1), (512, 6400, 4096, 1),
+          (900, 1000, 1400, 6)]
+
+
+@pytest.mark.parametrize("M,K,N,batch", RANDOM)
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+def test_split_error_no_larger_than_fp32(M, K, N, batch, ta, tb):
+    """N(0,1) operands. The error of a sum of K rounded terms is a random quantity; over the
+    >= 2.7 million outputs compared here its norm varies by less than 1 %, so 1.02 times the
+    fp32 kernel's is the bound for "no larger"."""
+    (a, lda, sA), (b, ldb, sB), a64, b64 = case(M, K, N, ta, tb, batch=batch, ints=False, seed=N)
+    c64 = a64 @ b64
+    err, outs = [], []
+    for direct in (0, 2):  # the dispatcher's choice, then the fp32 kernels
+        c = torch.full((batch, M, N), float("nan"), device="cuda:0")
+        with _native.tuned(direct=direct):
+            run(ta, tb, M, N, K, a, lda, sA, b, ldb, sB, None, c, N, M * N, batch)
+        err.append(float((c - c64).norm() / c64.norm()))
+        outs.append(c)
+    say("split error", M, K, N, batch, ta, tb, err)
+    assert not torch.equal(outs[0], outs[1]), "the call did not take the split kernel"
+    assert err[0] <= 1.02 * err[1]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+def test_split_nonfinite_and_tiny_operands(ta, tb):
+    """Infinities and NaN reach the outputs that fp32 arithmetic says, values below 2^-110
+    keep their precision, a value above bf16's rounding overflow stays finite, and every
+    other output is the exact product."""
+    M, K, N = 2100, 1009, 1300
+    (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, seed=5)
+
+    def put(x, t, i, k, value):  # element (i, k) of op(A), or (k, i) of op(B)
+        x.view(*((K, -1) if t else (-1, K)))[(k, i) if t else (i, k)] = value
+
+    put(a, ta, 7, 1000, float("inf"))
+    put(a, ta, 300, 3, float("nan"))
+    put(b, not tb, 1299, 500, float("-inf"))
+    a64[0, 7, 1000], a64[0, 300, 3], b64[0, 500, 1299] = np.inf, np.nan, -np.inf
+    put(a, ta, 1900, 16, 3.4e38)
+    b.view(*((N, K) if tb else (K, N)))[(slice(None), 16) if tb else 16] = 0.25
+    a64[0, 1900, 16], b64[0, 16, :] = float(np.float32(3.4e38)), 0.25
+    c = torch.empty(M, N, device="cuda:0")
+    say("split nonfinite", ta, tb)
+    run(ta, tb, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+    # (CPU: IEEE products one by one)
+    expect = torch.from_numpy(a64[0].cpu().numpy() @ b64[0].cpu().numpy()).float()
+    rows = torch.ones(M, dtype=torch.bool)
+    rows[1900] = False
+    got = c.cpu()
+    assert torch.equal(torch.nan_to_num(got[rows], nan=123.5), torch.nan_to_num(expect[rows], nan=123.5))
+    big = got[1900, :1299].double() / expect[1900, :1299].double()
+    assert bool(((big - 1).abs() < 1e-6).all())
+    # tiny: A of 2^-126 .. 2^-122, B scaled up by 2^60
+    (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, ints=False, seed=6)
+    a *= 2.0 ** -124
+    b *= 2.0 ** 60
+    a64 = (a.view(K, M).t() if ta else a.view(M, K)).double().contiguous()
+    b64 = (b.view(N, K).t() if tb else b.view(K, N)).double().contiguous()
+    run(ta, tb, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+    c64 = a64 @ b64
+    assert float((c.double() - c64).norm() / c64.norm()) < 1e-6  # fp32 chain: 5.7e-7
+
+
+def test_split_graph_capture_without_a_workspace():
+    """512 x 6400 x 4096 TN runs in more k ranges than the fp32 plan, which has one: captured
+    on a stream that holds no workspace it still runs, in one range, and replays agree."""
+    M, K, N = 512, 6400, 4096
+    (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, 1, 0, seed=9)
+    expect = (a64 @ b64)[0].float()
+    c = torch.full((M, N), float("nan"), device="cuda:0")
+    run(1, 0, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+    assert torch.equal(c, expect)
+    cap = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        run(1, 0, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+    for _ in range(3):
+        c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, expect)
