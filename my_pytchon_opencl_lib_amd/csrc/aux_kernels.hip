@@ -148,6 +148,103 @@ __global__ void __launch_bounds__(256) column_sum_kernel(const float *__restrict
         if (e < cnt) y[e] = accumulate ? y[e] + sum[e] : sum[e];
 }
 
+// Row sums (inner = 1): out[o] = sum over a of X[o][a], in column_sum_kernel's order (chunks
+// of CS_ROWS ascending from +0.0f, the chunk sums added in chunk order), so the bits are the
+// same. There every thread walked a row of its own, 4 bytes at a time at a stride of the row
+// length: 64000 rows of 513 (131 MB) took 135 us + 4.7 us for the chunk sums. Here a
+// wavefront owns a chunk of 64 rows and moves it through LDS in tiles of 64 columns: 16
+// loads of 16 bytes per lane cover 4 rows x 256 contiguous bytes each, the next tile's are in
+// flight while the lane of a row adds this tile's 64 values, 4 per LDS read (a row stride of
+// 68 floats keeps 16 lanes on distinct banks). The 4 wavefronts of a work-group take 4
+// consecutive chunks at a time and wavefront 0 adds their sums in order, so one launch does
+// all of it: 149 -> 28.9 us per call, 4.5 TB/s (4096 x 4096: 37 -> 17 us; 100 x 100000:
+// 42 -> 29). With few rows and many chunks (PARTIAL) each work-group takes
+// one group of 4 chunks and writes their sums [chunk][row] for reduce_slices_kernel.
+constexpr int CS_ROWS = 256;  // rows of the reduced axis per chunk
+constexpr int RS_TILE = 64;   // columns per tile (and rows per wavefront)
+constexpr int RS_LD = 68;
+
+template <bool PARTIAL>
+__global__ void __launch_bounds__(256) row_sum_kernel(const float *__restrict__ X,
+                                                      float *__restrict__ out, int outer,
+                                                      int axis) {
+    typedef float vec __attribute__((ext_vector_type(4)));
+    __shared__ __attribute__((aligned(16))) float tiles[4][RS_TILE * RS_LD];
+    __shared__ float sums[4][RS_TILE];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int o0 = blockIdx.x * RS_TILE;
+    const int chunks = (axis + CS_ROWS - 1) / CS_ROWS;
+    const int g0 = PARTIAL ? blockIdx.y * 4 : 0;
+    const int g1 = PARTIAL ? min(chunks, g0 + 4) : chunks;
+    float *tile = tiles[w];
+    // this lane's loads: 4 columns from 4 (lane % 16) of rows lane / 16 + 4 j
+    const int lc = 4 * (lane & 15);
+    const int lr = lane >> 4;
+    vec v[16];
+    auto fetch = [&](int c0, int c1) {  // columns c0 .. c0 + 63, those from c1 on zero
+        const bool whole = c0 + RS_TILE <= c1;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float *q = X + (int64_t)min(o0 + lr + 4 * j, outer - 1) * axis + c0 + lc;
+            if (whole) {
+                __builtin_memcpy(&v[j], q, sizeof(vec));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[j][e] = c0 + lc + e < c1 ? q[e] : 0.0f;
+            }
+        }
+    };
+    float total = 0.0f;
+    for (int g = g0; g < g1; g += 4) {
+        const int c = g + w;  // this wavefront's chunk
+        if (c < g1) {
+            const int a0 = c * CS_ROWS;
+            const int a1 = min(axis, a0 + CS_ROWS);
+            float sum = 0.0f;
+            fetch(a0, a1);
+            for (int a = a0; a < a1; a += RS_TILE) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    *reinterpret_cast<vec *>(tile + (lr + 4 * j) * RS_LD + lc) = v[j];
+                // (the wavefront's own LDS accesses complete in order; this keeps the compiler
+                // from moving them across)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (a + RS_TILE < a1) fetch(a + RS_TILE, a1);
+#pragma unroll
+                for (int q = 0; q < RS_TILE; q += 4) {
+                    const vec x = *reinterpret_cast<const vec *>(tile + lane * RS_LD + q);
+                    sum += x[0];
+                    sum += x[1];
+                    sum += x[2];
+                    sum += x[3];
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+            if constexpr (PARTIAL) {
+                if (o0 + lane < outer) out[(int64_t)c * outer + o0 + lane] = sum;
+            } else {
+                sums[w][lane] = sum;
+            }
+        }
+        if constexpr (!PARTIAL) {
+            __syncthreads();
+            if (w == 0) {
+                const int n = min(4, g1 - g);
+                total = g == 0 ? sums[0][lane] : total + sums[0][lane];
+                for (int q = 1; q < n; ++q) total += sums[q][lane];
+            }
+            __syncthreads();
+        }
+    }
+    if constexpr (!PARTIAL) {
+        const int o = o0 + lane;
+        if (w == 0 && o < outer) out[o] = total;
+    }
+}
+
 // Hp[t][h] = H[t - 1][h] when step t % seq_len > 0 of its sequence, else 0: the previous
 // hidden state of the same sequence, the left operand of grad_U += H_prev^T * grad_gates
 // (cs/cl_kernels/lstm.cl:582-590, tokens ordered [batch][seq_len]). VW consecutive h per
@@ -299,7 +396,7 @@ int launch_column_sum(hipStream_t stream, const float *X, float *Y, int outer, i
                       int inner, bool accumulate) {
     // Chunks of 256 rows: 12000 x 6565 (the Linear(500 -> 6565) bias gradient) is 47 chunks
     // of 7 work-groups, each thread with 16 rows of 128-bit loads in flight.
-    int rows = 256;
+    int rows = CS_ROWS;
     if ((axis + rows - 1) / rows > 65535) rows = (axis + 65534) / 65535;
     const int chunks = (axis + rows - 1) / rows;
     float *dst = Y;
@@ -308,6 +405,27 @@ int launch_column_sum(hipStream_t stream, const float *X, float *Y, int outer, i
         dst = static_cast<float *>(
             workspace(stream, (size_t)chunks * outer * inner * sizeof(float), &st));
         if (dst == nullptr) return st;
+    }
+    if (inner == 1 && !accumulate && rows == CS_ROWS && outer >= 64 && axis >= 16) {
+        // Rows shorter than 16 stay below: two lanes' worth of a tile. Fewer than 64 rows
+        // would leave lanes of every tile idle.
+        const int blocks = (outer + RS_TILE - 1) / RS_TILE;
+        // with 512 or more work-groups of rows, or one group of chunks, a work-group takes
+        // whole rows
+        const bool whole = chunks <= 4 || blocks >= 512;
+        if (whole)
+            MIGEMM_LAUNCH(row_sum_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, X,
+                          Y, outer, axis);
+        else
+            MIGEMM_LAUNCH(row_sum_kernel<true>,
+                          dim3((unsigned)blocks, (unsigned)((chunks + 3) / 4)), dim3(256), 0,
+                          stream, X, dst, outer, axis);
+        const int rc = launch_status("row_sum_kernel launch");
+        record_plan(PlanRecord{"row_sum", rows, RS_TILE, whole ? 1 : chunks, 16, outer, inner,
+                               axis, 1, false, false});
+        if (rc != MIGEMM_OK || whole) return rc;
+        return launch_reduce_slices(stream, dst, chunks, outer, 1, inner, nullptr, Y, inner,
+                                    inner);
     }
     const bool vec = inner % 4 == 0;
     const int64_t threads = (int64_t)outer * (vec ? inner / 4 : inner);
