@@ -13,7 +13,7 @@ NnClGlob.LinearForward) is the bias-epilogue form.
 import numpy as np
 import torch
 
-from .nncl_glob import NnClGlob, _require
+from .nncl_glob import NnClGlob, ShapeError, _require
 
 
 class Linear:
@@ -38,8 +38,8 @@ class Linear:
 
     def forward(self, x):
         """y[..., out] = x[..., in] @ weight^T, as one NT GEMM over all rows of x."""
-        _require(x.shape[-1] == self.in_features,
-                 f"x must end in {self.in_features} features (got {list(x.shape)})")
+        if x.shape[-1] != self.in_features:
+            raise ShapeError(f"x must end in {self.in_features} features (got {list(x.shape)})")
         x3 = x.reshape(1, -1, self.in_features).contiguous()  # layers.py:23-24
         y = self.nnclglob.BmmPermute(x3, self.weight.unsqueeze(0), transA=False, transB=True)
         return y.reshape(list(x.shape[:-1]) + [self.out_channels])  # :31-33
