@@ -1,7 +1,7 @@
 // Layout and reduction kernels of the matmul path:
-//  * tensor permute (cl_kernels/permute.cl:11-50): a batched 2-D transpose through LDS
-//    when the permutation swaps the last two axes (the [0,2,1] / [1,0] forms that
-//    BmmOp.Backward and the Python Linear use), else a generic <=10-D gather;
+//  * tensor permute (cl_kernels/permute.cl:11-50): through LDS tiles when the source's
+//    contiguous axis moves (the [0,2,1] / [1,0] forms that BmmOp.Backward and the Python
+//    Linear use among them), else a generic <=10-D gather;
 //  * column sums (cs/cl_kernels/linear.cl:149-168 linear_bias_backward and
 //    cs/cl_kernels/reduce_sum_axis.cl:3-24 reduce_sum_axis): each output is summed over
 //    the reduced axis in ascending order from +0.0f, exactly as the reference kernels do,
@@ -65,31 +65,99 @@ __global__ void __launch_bounds__(256) permute_gather_kernel(PermuteArgs a) {
     }
 }
 
-// dst[b][c][r] = src[b][r][c] for src [batch][R][Ccols]; 32x32 tiles through LDS with a
-// +1 pad so the column read of the tile is bank-conflict free.
-__global__ void __launch_bounds__(256) transpose_kernel(const float *__restrict__ src,
-                                                          float *__restrict__ dst, int R, int Cc,
-                                                          int tiles_c) {
-    __shared__ float tile[32][33];
-    const int b = blockIdx.y;
-    const int tr = blockIdx.x / tiles_c;
-    const int tc = blockIdx.x % tiles_c;
-    const int tx = threadIdx.x & 31;
-    const int ty = threadIdx.x >> 5;  // 0..7
-    const float *s = src + (int64_t)b * R * Cc;
-    float *d = dst + (int64_t)b * R * Cc;
+// dst[o][c][r] = src[row_offset(o, r) + c]: every permutation whose source-contiguous axis (c)
+// is not its innermost one. r runs over the destination axes behind c, merged (R of them,
+// contiguous in dst), o over those before it; row_offset unpacks both by invariant divisions.
+// A batched transpose is the case of one axis behind c.
+//  * HBM-bound: 64x64 tiles through LDS, 16 bytes per lane on both sides (no alignment
+//    needed), so a row of the tile is 256 contiguous bytes read and 256 written. LDS rows of
+//    65 floats keep the scalar writes and reads on distinct banks.
+//  * Consecutive work-groups of an XCD step along r: where dst rows do not start on 128-byte
+//    lines, neighbouring tiles share lines, and L2 merges the two parts before the line goes
+//    to HBM.
+// Measured (us per call, 3 rotating inputs, 32x32 tiles with 4-byte accesses or, for the
+// reversed axes, the gather kernel / this): 4096 x 4096 25.3 / 21.9 (6.1 TB/s), 4095 x 4097
+// 36.9 / 23.4, 64 x 600 x 600 by (0, 2, 1) 51.0 / 33.9, by (2, 1, 0) 175.9 / 38.4, 32 x 500
+// x 16 x 64 by (0, 2, 3, 1) 24.6 / 22.2.
+struct TransposeArgs {
+    const float *src;
+    float *dst;
+    uint32_t R, C;
+    uint32_t total;  // work-groups
+    FastDiv by_r, by_rc;
+    // source axes of r (innermost first) and of o (innermost first)
+    int nr, no;
+    FastDiv rdiv[MAXD], odiv[MAXD];
+    uint64_t rstride[MAXD], ostride[MAXD];
+};
+
+constexpr int TR = 64;  // tile edge
+
+__device__ __forceinline__ uint64_t unpack_offset(uint32_t t, int n, const FastDiv *div,
+                                                  const uint64_t *stride) {
+    uint64_t off = 0;
+    for (int i = 0; i + 1 < n; ++i) {
+        const uint32_t q = fast_div(t, div[i]);
+        off += (t - q * div[i].d) * stride[i];
+        t = q;
+    }
+    return off + t * stride[n - 1];
+}
+
+__global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
+    typedef float vec __attribute__((ext_vector_type(4)));
+    __shared__ float tile[TR][TR + 1];
+    uint32_t pid = blockIdx.x;
+    pid = (a.total & 7) == 0 ? (pid & 7) * (a.total >> 3) + (pid >> 3) : pid;
+    const uint32_t o = fast_div(pid, a.by_rc);
+    const uint32_t t = pid - o * a.by_rc.d;
+    const uint32_t tc = fast_div(t, a.by_r);
+    const uint32_t r0 = (t - tc * a.by_r.d) * TR;
+    const uint32_t c0 = tc * TR;
+    const uint64_t obase = a.no > 0 ? unpack_offset(o, a.no, a.odiv, a.ostride) : 0;
+    const uint32_t lane4 = 4 * (threadIdx.x & 15);  // this thread's 4 columns (rows of dst)
+    const uint32_t line = threadIdx.x >> 4;         // and its line of each 16
+    const uint32_t nr = min((uint32_t)TR, a.R - r0), nc = min((uint32_t)TR, a.C - c0);
+    const float *s = a.src + obase + c0;
+    vec v[4];
 #pragma unroll
-    for (int j = 0; j < 32; j += 8) {
-        const int r = tr * 32 + ty + j;
-        const int c = tc * 32 + tx;
-        if (r < R && c < Cc) tile[ty + j][tx] = s[(int64_t)r * Cc + c];
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t r = line + 16 * j;
+        if (r < nr) {
+            const float *q = s + unpack_offset(r0 + r, a.nr, a.rdiv, a.rstride) + lane4;
+            if (lane4 + 4 <= nc) {
+                __builtin_memcpy(&v[j], q, sizeof(vec));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[j][e] = lane4 + e < nc ? q[e] : 0.0f;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t r = line + 16 * j;
+        if (r < nr)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tile[r][lane4 + e] = v[j][e];
     }
     __syncthreads();
+    float *d = a.dst + ((size_t)o * a.C + c0) * a.R + r0;
 #pragma unroll
-    for (int j = 0; j < 32; j += 8) {
-        const int c = tc * 32 + ty + j;
-        const int r = tr * 32 + tx;
-        if (r < R && c < Cc) d[(int64_t)c * R + r] = tile[tx][ty + j];
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t c = line + 16 * j;
+        if (c < nc) {
+            vec x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = tile[lane4 + e][c];
+            float *q = d + (size_t)c * a.R + lane4;
+            if (lane4 + 4 <= nr) {
+                __builtin_memcpy(q, &x, sizeof(vec));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (lane4 + e < nr) q[e] = x[e];
+            }
+        }
     }
 }
 
@@ -343,24 +411,41 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
         cs[0] = 1;
         nd = 1;
     }
-    // Batched transpose of the last two axes with every leading axis in place: [R, C] ->
-    // [C, R] is dst axes (C: stride 1, R: stride C), leading batch axis of stride R * C.
-    const bool t2 = nd == 2 && cs[0] == 1 && cs[1] == cd[0];
-    const bool t3 = nd == 3 && cs[1] == 1 && cs[2] == cd[1] && cs[0] == cd[1] * cd[2];
-    if (t2 || t3) {
-        const int64_t batch = t3 ? cd[0] : 1;
-        const int64_t R = cd[nd - 1], Cc = cd[nd - 2];
-        const int64_t tiles_r = (R + 31) / 32;
-        const int64_t tiles_c = (Cc + 31) / 32;
-        if (batch <= 65535 && R <= INT32_MAX && Cc <= INT32_MAX &&
-            tiles_r * tiles_c <= INT32_MAX) {
-            MIGEMM_LAUNCH(transpose_kernel, dim3((unsigned)(tiles_r * tiles_c),
-                                                      (unsigned)batch),
-                               dim3(256), 0, stream, src, dst, (int)R, (int)Cc, (int)tiles_c);
-            record_plan(PlanRecord{"transpose", 32, 32, 1, 0, (int)R, (int)Cc, 0, (int)batch,
-                                   false, false});
-            return launch_status("transpose_kernel launch");
+    // The source's contiguous axis is not the innermost destination axis: through LDS tiles,
+    // unless a step of the axes before it holds fewer than 1024 elements, most of a tile then
+    // empty (us, gather / tiles: 64000 x 16 x 16 41.5 / 56.6, 200000 x 4 x 16 28.4 / 147.6,
+    // 20000 x 8 x 100 36.6 / 42.5; 4000 x 16 x 64 14.0 / 9.2, 20000 x 32 x 32 78.4 / 36.3).
+    int jc = 0;  // its place
+    while (cs[jc] != 1) ++jc;
+    int64_t behind = 1;  // elements per step of the axes before it
+    for (int i = jc; i < nd; ++i) behind *= cd[i];
+    int64_t R = 1;
+    for (int i = jc + 1; i < nd; ++i) R *= cd[i];
+    const int64_t outer = total / behind;
+    const int64_t tiles_r = (R + TR - 1) / TR, tiles_c = (cd[jc] + TR - 1) / TR;
+    if (jc < nd - 1 && (jc == 0 || behind >= 1024) && R <= INT32_MAX && cd[jc] <= INT32_MAX &&
+        outer * tiles_r * tiles_c <= INT32_MAX) {
+        TransposeArgs a;
+        a.src = src;
+        a.dst = dst;
+        a.nr = a.no = 0;
+        for (int i = nd - 1; i > jc; --i, ++a.nr) {
+            a.rdiv[a.nr] = make_fastdiv((uint32_t)cd[i]);
+            a.rstride[a.nr] = (uint64_t)cs[i];
         }
+        for (int i = jc - 1; i >= 0; --i, ++a.no) {
+            a.odiv[a.no] = make_fastdiv((uint32_t)cd[i]);
+            a.ostride[a.no] = (uint64_t)cs[i];
+        }
+        a.R = (uint32_t)R;
+        a.C = (uint32_t)cd[jc];
+        a.by_r = make_fastdiv((uint32_t)tiles_r);
+        a.by_rc = make_fastdiv((uint32_t)(tiles_r * tiles_c));
+        a.total = (uint32_t)(outer * tiles_r * tiles_c);
+        MIGEMM_LAUNCH(transpose_kernel, dim3(a.total), dim3(256), 0, stream, a);
+        record_plan(PlanRecord{"transpose", TR, TR, 1, 16, (int)a.R, (int)a.C, 0, (int)outer,
+                               false, false});
+        return launch_status("transpose_kernel launch");
     }
     // 16-byte elements when the innermost destination axis is the source's contiguous one
     // and holds whole groups of 4 (every other stride is then a multiple of 4 as well)
