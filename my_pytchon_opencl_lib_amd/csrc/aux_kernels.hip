@@ -72,9 +72,10 @@ __global__ void __launch_bounds__(256) permute_gather_kernel(PermuteArgs a) {
 //  * HBM-bound: 64x64 tiles through LDS, 16 bytes per lane on both sides (no alignment
 //    needed), so a row of the tile is 256 contiguous bytes read and 256 written. LDS rows of
 //    65 floats keep the scalar writes and reads on distinct banks.
-//  * Consecutive work-groups of an XCD step along r: where dst rows do not start on 128-byte
-//    lines, neighbouring tiles share lines, and L2 merges the two parts before the line goes
-//    to HBM.
+//  * Consecutive work-groups of an XCD step along r, in groups of 32 tiles: where dst rows do
+//    not start on 128-byte lines, neighbouring tiles share lines, and L2 merges the two parts
+//    before the line goes to HBM. Whole columns of tiles would touch every page of a large
+//    source at once (46342 x 46342: 7036 us, in groups 6300).
 // Measured (us per call, 3 rotating inputs, 32x32 tiles with 4-byte accesses or, for the
 // reversed axes, the gather kernel / this): 4096 x 4096 25.3 / 21.9 (6.1 TB/s), 4095 x 4097
 // 36.9 / 23.4, 64 x 600 x 600 by (0, 2, 1) 51.0 / 33.9, by (2, 1, 0) 175.9 / 38.4, 32 x 500
@@ -83,15 +84,19 @@ struct TransposeArgs {
     const float *src;
     float *dst;
     uint32_t R, C;
+    uint32_t tiles_r;
     uint32_t total;  // work-groups
-    FastDiv by_r, by_rc;
+    FastDiv by_rc;       // tiles_r * tiles_c
+    FastDiv in_group;    // TR_GROUP * tiles_c
+    FastDiv last_group;  // tiles of r in the last group
     // source axes of r (innermost first) and of o (innermost first)
     int nr, no;
     FastDiv rdiv[MAXD], odiv[MAXD];
     uint64_t rstride[MAXD], ostride[MAXD];
 };
 
-constexpr int TR = 64;  // tile edge
+constexpr int TR = 64;        // tile edge
+constexpr int TR_GROUP = 32;  // tiles of r rastered together
 
 __device__ __forceinline__ uint64_t unpack_offset(uint32_t t, int n, const FastDiv *div,
                                                   const uint64_t *stride) {
@@ -111,8 +116,17 @@ __global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
     pid = (a.total & 7) == 0 ? (pid & 7) * (a.total >> 3) + (pid >> 3) : pid;
     const uint32_t o = fast_div(pid, a.by_rc);
     const uint32_t t = pid - o * a.by_rc.d;
-    const uint32_t tc = fast_div(t, a.by_r);
-    const uint32_t r0 = (t - tc * a.by_r.d) * TR;
+    const uint32_t first = fast_div(t, a.in_group) * TR_GROUP;
+    const uint32_t tg = t - first / TR_GROUP * a.in_group.d;
+    uint32_t tc, tr;
+    if (a.tiles_r - first >= TR_GROUP) {
+        tc = tg / TR_GROUP;
+        tr = first + tg % TR_GROUP;
+    } else {
+        tc = fast_div(tg, a.last_group);
+        tr = first + tg - tc * a.last_group.d;
+    }
+    const uint32_t r0 = tr * TR;
     const uint32_t c0 = tc * TR;
     const uint64_t obase = a.no > 0 ? unpack_offset(o, a.no, a.odiv, a.ostride) : 0;
     const uint32_t lane4 = 4 * (threadIdx.x & 15);  // this thread's 4 columns (rows of dst)
@@ -424,7 +438,7 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
     const int64_t outer = total / behind;
     const int64_t tiles_r = (R + TR - 1) / TR, tiles_c = (cd[jc] + TR - 1) / TR;
     if (jc < nd - 1 && (jc == 0 || behind >= 1024) && R <= INT32_MAX && cd[jc] <= INT32_MAX &&
-        outer * tiles_r * tiles_c <= INT32_MAX) {
+        outer * tiles_r * tiles_c <= INT32_MAX && TR_GROUP * tiles_c <= INT32_MAX) {
         TransposeArgs a;
         a.src = src;
         a.dst = dst;
@@ -439,7 +453,9 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
         }
         a.R = (uint32_t)R;
         a.C = (uint32_t)cd[jc];
-        a.by_r = make_fastdiv((uint32_t)tiles_r);
+        a.tiles_r = (uint32_t)tiles_r;
+        a.in_group = make_fastdiv((uint32_t)(TR_GROUP * tiles_c));
+        a.last_group = make_fastdiv((uint32_t)(tiles_r % TR_GROUP));
         a.by_rc = make_fastdiv((uint32_t)(tiles_r * tiles_c));
         a.total = (uint32_t)(outer * tiles_r * tiles_c);
         MIGEMM_LAUNCH(transpose_kernel, dim3(a.total), dim3(256), 0, stream, a);

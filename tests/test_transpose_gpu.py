@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape", [(1, 65), (64, 64), (63, 129), (200, 3), (5, 64, 65),
-                                   (70, 1, 130), (129, 3, 66), (2, 127, 40), (3, 65, 2, 70),
+                                   (70, 1, 130), (2200, 70), (129, 3, 66), (2, 127, 40), (3, 65, 2, 70),
                                    (7, 5, 64, 33), (66, 4, 3, 5), (2, 3, 4, 5, 130)])
 def test_every_permutation(nncl, shape):
     n = 1
