@@ -47,19 +47,33 @@ namespace migemm {
 
 namespace {
 
-// One k-tile (16 k) of a tile costs a CU `full` us when every CU works (the power limit)
-// and `alone` us when the CU has one work-group and the chip is not full; `over` us per
-// tile on each CU for the first loads, the C store and the launch of the next work-group.
-// Fitted to 4096^3, 2048^3, 1024^3, 6400 x 512 x 4096, 12000 x 500 x 6565, 1024 x 1024 x
-// 4096 and the k-split gradients 12000 x 6565 x 500 and 500 x 12000 x 6565 (+-6 %).
+// Estimated time of `t` x 256 tiles (us per k-tile of 16, without the tiles' fixed part).
+// A work-group that has its CU to itself takes `full` us per k-tile when every CU works (the
+// power limit) and `alone` when few do; a last, partial round lies between. 128x128 tiles
+// run two to a CU: up to 8 rounds each CU's share is a whole number of them, beyond that
+// they even out.
 struct SplitFit {
     int bm, bn;
-    double full, alone, over;
+    double full, alone, over;  // over: us per tile and CU for first loads, C store, launch
 };
+// Fitted on one box (events around 10 launches; estimate / measured, us): 4096^3 256x256
+// 627 / 605-650; 6400 x 2048 x 4096 256x256 613 / 584, 128x128 653 / 611; 2048^3 128x128
+// 103 / 100; 1000 x 777 x 3000 128x128 42 / 41; 500 x 12000 x 6565 TN in 6 ranges 256x128
+// 505 / 488, 128x128 459 / 490, in 5 ranges 582 / 564, 547 / 534.
 constexpr SplitFit kSplitFit[3] = {
-    {256, 256, 2.44, 1.80, 20.0}, {256, 128, 1.38, 1.05, 11.0}, {128, 128, 0.72, 0.60, 3.5}};
-constexpr double kSplitLaunch = 5.0;          // us: start of the grid
-constexpr double kSplitPartialBytes = 6e6;    // partial sums' HBM traffic, bytes per us
+    {256, 256, 2.35, 1.75, 20.0}, {256, 128, 1.29, 1.05, 11.0}, {128, 128, 0.70, 0.58, 3.5}};
+constexpr double kSplitLaunch = 5.0;        // us: start of the grid
+constexpr double kSplitPartialBytes = 6e6;  // partial sums' HBM traffic, bytes per us
+// C rows off 64-byte boundaries: us more per tile and CU (12000 x 500 x 6565 against x 6560:
+// 256x256 532 / 474, 128x128 508 / 486)
+constexpr double kSplitOddRows[3] = {11.0, 5.0, 1.2};
+
+double split_rounds(const SplitFit &f, double t) {
+    const double whole = floor(t), part = t - whole;
+    if (f.bn == 128 && f.bm == 128)
+        return t <= 1 ? f.alone + 0.12 * t : (t <= 8 ? ceil(t) : t + 0.3) * f.full;
+    return whole * f.full + (part > 0 ? f.alone + (f.full - f.alone) * part : 0.0);
+}
 
 }  // namespace
 
@@ -72,7 +86,10 @@ SplitPlan plan_split(const GemmDesc &d, int plan_splits) {
     const int least = (77 * plan_splits + 99) / 100;
     const int most = plan_splits > 8 ? plan_splits : 8;
     const int nk = (d.K + SBK - 1) / SBK;
-    for (const SplitFit &f : kSplitFit) {
+    const bool odd = d.ldc % 16 != 0 || ((uintptr_t)d.C & 63) != 0 ||
+                     (d.batch > 1 && d.sC % 16 != 0);
+    for (int i = 0; i < 3; ++i) {
+        const SplitFit &f = kSplitFit[i];
         const double tiles =
             (double)((d.M + f.bm - 1) / f.bm) * ((d.N + f.bn - 1) / f.bn) * d.batch;
         for (int s = least; s <= most; ++s) {
@@ -83,8 +100,9 @@ SplitPlan plan_split(const GemmDesc &d, int plan_splits) {
             const double ks = (double)((nk + s - 1) / s);
             if (s > 1 && ks < 16) break;
             const double t = tiles * s / 256.0;
-            const double us = ks * fmax(t * f.full, ceil(t) * f.alone) +
-                              fmax(t, 1.0) * f.over + kSplitLaunch +
+            const double over = f.over + (odd && s == 1 ? kSplitOddRows[i] : 0.0);
+            const double us = ks * split_rounds(f, t) +
+                              (f.bm == 256 ? ceil(t) : fmax(t, 1.0)) * over + kSplitLaunch +
                               (s > 1 ? (2.0 * partial + 4.0 * d.batch * d.M * d.N) /
                                                kSplitPartialBytes + 4.0
                                      : 0.0);

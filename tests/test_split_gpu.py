@@ -51,8 +51,8 @@ def case(M, K, N, ta, tb, batch=1, pad=0, off=0, ints=True, seed=0):
     return (a, lda, sA), (b, ldb, sB), a64, b64
 
 
-# 128x128 (2100 x 1009 x 1300), 256x128 and 256x256 tiles; K % 16 = 0, 1, 15 and 9
-SHAPES = [(2100, 1009, 1300), (4097, 144, 3073), (5000, 511, 2049), (3073, 2048, 4225)]
+# 128x128 (2100 x 1009 x 1900), 256x128 and 256x256 tiles; K % 16 = 0, 1, 15 and 9
+SHAPES = [(2100, 1009, 1900), (4097, 144, 3073), (5000, 511, 2049), (3073, 2048, 4225)]
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
@@ -77,9 +77,9 @@ def test_split_exact(M, K, N, ta, tb):
 
 # (M, K, N, batch): one range; k ranges as the fp32 plan has them (6400 x 4096 x 512 in 3,
 # 500 x 12000 x 6565 in 6); more ranges than it has (512 x 6400 x 4096); a batch
-RANDOM = [(2100, 1009, 1300, 1), (4096, 512, 3000, 1), (4096, 2048, 4096, 1),
+RANDOM = [(2100, 1009, 1900, 1), (4096, 512, 3000, 1), (4096, 2048, 4096, 1),
           (6400, 4096, 512, 1), (500, 12000, 6565, 1), (512, 6400, 4096, 1),
-          (900, 1000, 1400, 6)]
+          (900, 1000, 1400, 8)]
 
 
 @pytest.mark.parametrize("M,K,N,batch", RANDOM)
@@ -107,7 +107,7 @@ def test_split_nonfinite_and_tiny_operands(ta, tb):
     """Infinities and NaN reach the outputs that fp32 arithmetic says, values below 2^-110
     keep their precision, a value above bf16's rounding overflow stays finite, and every
     other output is the exact product."""
-    M, K, N = 2100, 1009, 1300
+    M, K, N = 2100, 1009, 1900
     (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, seed=5)
 
     def put(x, t, i, k, value):  # element (i, k) of op(A), or (k, i) of op(B)
@@ -115,8 +115,8 @@ def test_split_nonfinite_and_tiny_operands(ta, tb):
 
     put(a, ta, 7, 1000, float("inf"))
     put(a, ta, 300, 3, float("nan"))
-    put(b, not tb, 1299, 500, float("-inf"))
-    a64[0, 7, 1000], a64[0, 300, 3], b64[0, 500, 1299] = np.inf, np.nan, -np.inf
+    put(b, not tb, 1899, 500, float("-inf"))
+    a64[0, 7, 1000], a64[0, 300, 3], b64[0, 500, 1899] = np.inf, np.nan, -np.inf
     put(a, ta, 1900, 16, 3.4e38)
     b.view(*((N, K) if tb else (K, N)))[(slice(None), 16) if tb else 16] = 0.25
     a64[0, 1900, 16], b64[0, 16, :] = float(np.float32(3.4e38)), 0.25
@@ -129,7 +129,7 @@ def test_split_nonfinite_and_tiny_operands(ta, tb):
     rows[1900] = False
     got = c.cpu()
     assert torch.equal(torch.nan_to_num(got[rows], nan=123.5), torch.nan_to_num(expect[rows], nan=123.5))
-    big = got[1900, :1299].double() / expect[1900, :1299].double()
+    big = got[1900, :1899].double() / expect[1900, :1899].double()
     assert bool(((big - 1).abs() < 1e-6).all())
     # tiny: A of 2^-126 .. 2^-122, B scaled up by 2^60
     (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, ints=False, seed=6)
