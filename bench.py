@@ -46,11 +46,17 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3  # MI355X dense FP32 matrix peak (AMD public specification)
 PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
+# gemm_split_kernel computes each fp32 product as six bf16 products on the bf16 MFMA (2516.6
+# TFLOP/s dense), so its roofline peak in fp32 FLOP is a sixth of that rate
+PEAK_SPLIT_TFLOPS = round(2516.6 / 6, 1)
 N4096 = 4096
 FLOP_4096 = 2.0 * N4096 ** 3
 EVENT_EVERY = 2  # timed steps per step whose launches carry HIP events
 TRACE_SUMMARY = os.path.join(ROOT, "profiles", "gemm_direct_4096_kernel_trace.md")
 PMC_SUMMARY = os.path.join(ROOT, "profiles", "gemm_direct_4096_pmc.md")
+# the same of gemm_split_kernel, which runs the three forms
+SPLIT_TRACE_SUMMARY = os.path.join(ROOT, "profiles", "gemm_split_4096_kernel_trace.md")
+SPLIT_PMC_SUMMARY = os.path.join(ROOT, "profiles", "gemm_split_4096_pmc.md")
 # GPU box: one GPU's share of the host is 16 threads (OMP_NUM_THREADS there)
 CPU_SHARE = 16
 
@@ -309,11 +315,12 @@ def main():
     ref = None if args.no_reference else reference_same_gpu(per_form["NN"]["ms"])
     cpu = None if args.no_cpu_baseline else cpu_baseline(args.cpu_seconds)
 
-    prof = load_profiled()
-    roofline = {"bound": "mfma", "kernel": f"gemm_direct_kernel ({dominant} form, 256x256 tiles)",
-                "achieved": round(achieved, 3), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4),
-                "traffic": load_traffic(dominant),
+    prof = load_profiled(SPLIT_TRACE_SUMMARY)
+    roofline = {"bound": "mfma", "kernel": f"gemm_split_kernel ({dominant} form, 256x256 tiles)",
+                "achieved": round(achieved, 3), "peak": PEAK_SPLIT_TFLOPS,
+                "unit": "TFLOP/s", "frac": round(achieved / PEAK_SPLIT_TFLOPS, 4),
+                "peak_is": "dense bf16 MFMA rate / 6 (bf16 products per fp32 product)",
+                "traffic": load_traffic(dominant, SPLIT_PMC_SUMMARY),
                 "algorithmic_per_launch": {"flop": FLOP_4096, "bytes": 4 * 3 * n * n},
                 "measured_by": f"HIP events around each launch of one timed step in "
                                f"{EVENT_EVERY}, on the launch stream, this run"}
@@ -321,10 +328,10 @@ def main():
         pus = prof[dominant]
         roofline["profiled_us"] = pus
         roofline["frac_profiled"] = round(FLOP_4096 / (pus * 1e-6) / 1e12 /
-                                          PEAK_FP32_MFMA_TFLOPS, 4)
-        roofline["profile"] = "profiles/gemm_direct_4096_kernel_trace.md (timed launches " \
+                                          PEAK_SPLIT_TFLOPS, 4)
+        roofline["profile"] = "profiles/gemm_split_4096_kernel_trace.md (timed launches " \
                               "under rocprofv3 --kernel-trace)"
-    roofline["traffic_source"] = "profiles/gemm_direct_4096_pmc.md (rocprofv3 --pmc " \
+    roofline["traffic_source"] = "profiles/gemm_split_4096_pmc.md (rocprofv3 --pmc " \
                                  "FETCH_SIZE + WRITE_SIZE, copy-kernel scaled)"
 
     line = {
@@ -422,13 +429,13 @@ def pmc_target(torch, nncl, which="4096"):
     print(f"pmc target {which} done", flush=True)
 
 
-def load_traffic(form):
+def load_traffic(form, path=PMC_SUMMARY):
     """HBM bytes per launch measured by rocprofv3 --pmc (FETCH_SIZE + WRITE_SIZE, each
     scaled by the copy-kernel factor) for the dominant form, from the committed profile
     summary; None when no summary covers it."""
-    if not os.path.exists(PMC_SUMMARY):
+    if not os.path.exists(path):
         return None
-    for line in open(PMC_SUMMARY):
+    for line in open(path):
         if line.startswith("TRAFFIC_BYTES_PER_LAUNCH"):
             _, f, nbytes = line.split()[:3]
             if f == form:
@@ -436,12 +443,12 @@ def load_traffic(form):
     return None
 
 
-def load_profiled():
+def load_profiled(path=TRACE_SUMMARY):
     """Timed-launch average duration (us) of each 4096^3 form under rocprofv3, from the
     committed kernel-trace summary of this bench."""
     out = {}
-    if os.path.exists(TRACE_SUMMARY):
-        for line in open(TRACE_SUMMARY):
+    if os.path.exists(path):
+        for line in open(path):
             if line.startswith("PROFILED_US"):
                 _, f, us = line.split()[:3]
                 out[f] = float(us)
@@ -473,7 +480,8 @@ def summarize_trace(directory, steps, warmup):
         short = short.replace("void ", "")
         us = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
         by_kernel.setdefault(short, []).append(us)
-        m = re.search(r"gemm_direct_kernel<256, 256, \d+, \d+, (true|false), (true|false)", name)
+        m = re.search(r"gemm_(?:direct|split)_kernel<256, 256, \d+, \d+, "
+                      r"(true|false), (true|false)", name)
         if m:
             forms.setdefault(FORM_OF[m.groups()], []).append(us)
     print("| kernel | launches | average (us) | min (us) | max (us) |")
