@@ -377,6 +377,9 @@ int migemm_set_gemm_policy(int policy, int *previous);
 #define MIGEMM_TUNE_SMALL_TILES 4  /* small-output kernel's 32x32 tiles: 1 never,
                                       2 always (M, N > 16) */
 #define MIGEMM_TUNE_SMALL_SPLITK 5 /* small-output kernel's k ranges: S in 1..64 */
+#define MIGEMM_TUNE_PLAN_WORKSPACE 6 /* KiB of workspace that migemm_gemm_plan assumes, as
+                                      for a stream that is being captured (0: as much as
+                                      the call asks for); real calls ignore it */
 #define MIGEMM_TILE_128x256 128256
 int migemm_set_tuning(int key, int value, int *previous);
 

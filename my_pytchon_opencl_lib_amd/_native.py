@@ -36,10 +36,12 @@ MIGEMM_TUNE_SPLITK = 2
 MIGEMM_TUNE_DIRECT = 3
 MIGEMM_TUNE_SMALL_TILES = 4
 MIGEMM_TUNE_SMALL_SPLITK = 5
+MIGEMM_TUNE_PLAN_WORKSPACE = 6
 MIGEMM_TILE_128x256 = 128256
 TUNE_KEYS = {"tile": MIGEMM_TUNE_TILE, "splitk": MIGEMM_TUNE_SPLITK,
              "direct": MIGEMM_TUNE_DIRECT, "small_tiles": MIGEMM_TUNE_SMALL_TILES,
-             "small_splitk": MIGEMM_TUNE_SMALL_SPLITK}
+             "small_splitk": MIGEMM_TUNE_SMALL_SPLITK,
+             "plan_workspace": MIGEMM_TUNE_PLAN_WORKSPACE}
 
 STATUS_NAMES = {
     MIGEMM_OK: "MIGEMM_OK",

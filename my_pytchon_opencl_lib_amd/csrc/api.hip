@@ -117,6 +117,12 @@ int stream_device(hipStream_t stream, int *device) {
 // by running the same call once on that stream outside the capture.
 void *workspace(hipStream_t stream, size_t bytes, int *status, int slot) {
     if (t_plan_only) {
+        const size_t held = (size_t)tuning(MIGEMM_TUNE_PLAN_WORKSPACE) << 10;
+        if (held != 0 && bytes > held) {
+            *status = set_error(MIGEMM_ERR_WORKSPACE, "%zu bytes of workspace are needed but a "
+                                "dry run has %zu (MIGEMM_TUNE_PLAN_WORKSPACE)", bytes, held);
+            return nullptr;
+        }
         *status = MIGEMM_OK;
         return kPlanPlaceholder;
     }
@@ -310,7 +316,7 @@ static int validate_gemm(int transA, int transB, int M, int N, int K, const floa
 // Kernel-family policy (migemm_set_gemm_policy) and tuning overrides (migemm_set_tuning),
 // process-wide.
 static std::atomic<int> g_policy{MIGEMM_POLICY_AUTO};
-static std::atomic<int> g_tuning[MIGEMM_TUNE_SMALL_SPLITK + 1];
+static std::atomic<int> g_tuning[MIGEMM_TUNE_PLAN_WORKSPACE + 1];
 
 int tuning(int key) { return g_tuning[key].load(std::memory_order_relaxed); }
 
@@ -930,6 +936,7 @@ int migemm_set_tuning(int key, int value, int *previous) {
         case MIGEMM_TUNE_SMALL_SPLITK: ok = value >= 0 && value <= 64; break;
         case MIGEMM_TUNE_DIRECT:
         case MIGEMM_TUNE_SMALL_TILES: ok = value >= 0 && value <= 2; break;
+        case MIGEMM_TUNE_PLAN_WORKSPACE: ok = value >= 0; break;
         default:
             return set_error(MIGEMM_ERR_INVALID_ARG, "set_tuning: unknown key %d", key);
     }

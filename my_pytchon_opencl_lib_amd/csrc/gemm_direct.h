@@ -387,6 +387,7 @@ int launch_direct(hipStream_t s, TiledArgs &a) {
         return set_error(MIGEMM_ERR_UNSUPPORTED, "gemm: %lld tiles exceed one launch",
                          (long long)total);
     a.total = (int)total;
+    if (const int rc = check_partials(a)) return rc;
     set_tile_divisors(a);
     MIGEMM_LAUNCH((gemm_direct_kernel<BM, BN, WM, WN, AKC, BKC, BK, S, D, OCC, WA, WB>),
                        dim3(a.total),

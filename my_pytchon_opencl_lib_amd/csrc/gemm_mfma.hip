@@ -476,6 +476,7 @@ int launch_tiles(hipStream_t s, TiledArgs &a, bool akc, bool bkc, bool av, bool 
         return set_error(MIGEMM_ERR_UNSUPPORTED, "gemm: %lld tiles exceed one launch",
                          (long long)total);
     a.total = (int)total;
+    if (const int rc = check_partials(a)) return rc;
     set_tile_divisors(a);
     if constexpr (ONLY >= 0)
         return launch_vec<BM, BN, BK, WM, WN, (ONLY >> 1) != 0, (ONLY & 1) != 0>(s, a, av, bv);
@@ -869,22 +870,25 @@ int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d, bool automatic) {
     // (tiled_common.h, store_tile)
     a.write_back = cfg == 128 && !rows64;
     a.partial = nullptr;
-    if (splits > 1) {
-        int st = MIGEMM_OK;
-        a.partial =
-            partial_buffer(stream, d, (size_t)splits * d.batch * d.M * d.N * sizeof(float), &st);
-        if (a.partial == nullptr) return st;
-    }
-    if (split_plan.bm != 0 && split_plan.splits > splits) {
-        // more k ranges than the plan's: where their partial sums are not to be had (a
-        // stream being captured without a workspace), the plan runs as it is
-        int st = MIGEMM_OK;
-        a.partial = partial_buffer(
-            stream, d, (size_t)split_plan.splits * d.batch * d.M * d.N * sizeof(float), &st);
+    // Room for the partial sums of the plan that is to run, asked for once. Where the split
+    // kernel's are not to be had (a stream being captured whose workspace holds the fp32
+    // plan's fewer ranges, or none; device memory that holds only those), the fp32 plan runs.
+    auto partials = [&](int ranges, int *st) {
+        return partial_buffer(stream, d, (size_t)ranges * d.batch * d.M * d.N * sizeof(float),
+                              st);
+    };
+    int st = MIGEMM_OK;
+    if (split_plan.bm != 0 && split_plan.splits > 1) {
+        a.partial = partials(split_plan.splits, &st);
         if (a.partial == nullptr) {
+            if (st != MIGEMM_ERR_WORKSPACE) return st;
             clear_error();
             split_plan.bm = 0;
         }
+    }
+    if (split_plan.bm == 0 && splits > 1) {
+        a.partial = partials(splits, &st);
+        if (a.partial == nullptr) return st;
     }
     if (split_plan.bm != 0) {
         TiledArgs sa = a;

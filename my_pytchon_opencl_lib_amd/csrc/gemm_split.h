@@ -362,6 +362,7 @@ int launch_split(hipStream_t s, TiledArgs &a) {
         return set_error(MIGEMM_ERR_UNSUPPORTED, "gemm: %lld tiles exceed one launch",
                          (long long)total);
     a.total = (int)total;
+    if (const int rc = check_partials(a)) return rc;
     set_tile_divisors(a);
     MIGEMM_LAUNCH((gemm_split_kernel<BM, BN, WM, WN, AKC, BKC>), dim3(a.total),
                   dim3(WM * WN * 64), 0, s, a);

@@ -274,9 +274,12 @@ int devmem_alloc_on(hipStream_t stream, int device, size_t bytes, void **ptr) {
     if (rc != MIGEMM_OK) return rc;
     void *p = nullptr;
     hipError_t e = hipMallocFromPoolAsync(&p, bytes, m->pool, stream);
-    if (e == hipErrorOutOfMemory)
+    if (e == hipErrorOutOfMemory) {
+        // reported here: the caller may go on with less, whose launch status is its own
+        (void)hipGetLastError();
         return set_error(MIGEMM_ERR_WORKSPACE, "workspace of %zu bytes: out of device memory",
                          bytes);
+    }
     MIGEMM_HIP(e);
     *ptr = p;
     return MIGEMM_OK;

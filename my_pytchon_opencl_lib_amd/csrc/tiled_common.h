@@ -47,6 +47,14 @@ inline void set_tile_divisors(TiledArgs &a) {
     a.last_group = make_fastdiv((uint32_t)(rem == 0 ? TILE_GROUP : rem));
 }
 
+// Checked by every launcher of k ranges: their partial sums need a buffer.
+inline int check_partials(const TiledArgs &a) {
+    if (a.splits > 1 && a.partial == nullptr)
+        return set_error(MIGEMM_ERR_WORKSPACE, "gemm: %d k ranges without a buffer for their "
+                         "partial sums", a.splits);
+    return MIGEMM_OK;
+}
+
 struct TileCoord {
     int split, b, m0, n0;
 };

@@ -4,6 +4,8 @@ nothing, makes no HIP call): every BASELINE config, every caller shape of the pa
 regime table (tests/dispatch_cases.py). A change to the dispatcher shows up here as a
 changed plan string; the GPU suite checks that real calls record the same plans
 (tests/test_gemm_gpu.py::test_dry_run_plans_match_real_calls)."""
+import random
+
 import pytest
 
 import dispatch_cases as dc
@@ -52,3 +54,49 @@ def test_plan_follows_policy_and_tuning():
     with _native.tuned(tile=128, splitk=2):
         assert _native.gemm_plan(*a).startswith("tiled-direct tile=128x128 splits=2 ")
     assert _native.gemm_plan(*a).startswith("tiled-direct tile=256x256 splits=1 ")
+
+
+# (M, K, N, ta, tb, k ranges of the fp32 plan): products whose split plan has more ranges
+PARTIALS = [(960, 4736, 704, 1, 0, 4), (1536, 4096, 3072, 0, 1, 2), (640, 1472, 1280, 0, 0, 4),
+            (6400, 4096, 512, 0, 1, 3), (512, 6400, 4096, 1, 0, 1)]
+
+
+@pytest.mark.parametrize("M,K,N,ta,tb,ranges", PARTIALS)
+def test_partial_sums_fit_the_workspace_or_another_plan_runs(M, K, N, ta, tb, ranges):
+    """With a workspace that holds the fp32 plan's partial sums but not the split plan's (a
+    stream being captured) the fp32 plan runs in that workspace; with less, the call is
+    refused. A launch of k ranges without a buffer for them is an error in any plan."""
+    a = dc.args(M, N, K, ta=ta, tb=tb)
+    fp32 = ranges * M * N * 4 if ranges > 1 else 0
+    free = _native.gemm_plan(*a)
+    for kib in (-(-fp32 // 1024) or 1, 1 << 20):
+        with _native.tuned(plan_workspace=kib):
+            plan = _native.gemm_plan(*a)
+        if kib < 1 << 20:
+            assert f"splits={ranges} " in plan
+        else:
+            assert plan == free
+    if ranges > 1:
+        with _native.tuned(plan_workspace=fp32 // 1024 - 1):
+            with pytest.raises(_native.MigemmRuntimeError, match="bytes of workspace are needed"):
+                _native.gemm_plan(*a)
+
+
+def test_no_plan_launches_k_ranges_without_a_buffer():
+    """Products over the tiled family's range, each under workspaces of 1 KiB to 1 GiB: the
+    dispatcher plans a launch or refuses for want of workspace, and what runs in a workspace
+    runs in any larger one."""
+    rng = random.Random(5)
+    for _ in range(400):
+        M, K, N = (rng.randrange(200, 6500) // 32 * 32 + rng.choice([0, 0, 1]) for _ in range(3))
+        a = dc.args(M, N, K, ta=rng.randrange(2), tb=rng.randrange(2))
+        ran = False
+        for kib in [1 << e for e in range(0, 21, 2)]:
+            with _native.tuned(plan_workspace=kib):
+                try:
+                    _native.gemm_plan(*a)
+                    ran = True
+                except _native.MigemmRuntimeError as e:
+                    assert "bytes of workspace are needed" in str(e)
+                    assert not ran, (M, K, N, a[:2], kib)
+        assert ran, (M, K, N, a[:2])

@@ -162,3 +162,31 @@ def test_split_graph_capture_without_a_workspace():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, expect)
+
+
+def test_split_graph_capture_in_a_workspace_for_fewer_ranges():
+    """6400 x 4096 x 512 NT: 3 k ranges on the fp32 MFMA, more in the split kernel. A capture
+    on a stream that reserved room for the 3 runs those in it; replays agree with fp64."""
+    M, K, N = 6400, 4096, 512
+    (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, 0, 1, seed=11)
+    expect = (a64 @ b64)[0].float()
+    c = torch.full((M, N), float("nan"), device="cuda:0")
+    cap = torch.cuda.Stream()
+    held = ctypes.c_size_t(0)
+    s = ctypes.c_void_p(cap.cuda_stream)
+    _native.call("migemm_workspace_reserve", s, 3 * M * N * 4)
+    _native.call("migemm_workspace_size", s, ctypes.byref(held))
+    assert 3 * M * N * 4 <= held.value < 5 * M * N * 4
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        run(0, 1, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+    assert "splits=3 " in _native.last_plan()
+    say("replay in 3 ranges")
+    for _ in range(3):
+        c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, expect)
+    _native.call("migemm_workspace_release", s)
