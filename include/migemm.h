@@ -386,9 +386,8 @@ int migemm_set_tuning(int key, int value, int *previous);
 /* Writes a one-line description of the kernel the last GEMM / permute / column-sum call of
  * this host thread ran (family, output tile, k ranges, load width, shape, layout) into
  * buf (NUL-terminated, truncated to len). For tests and tuning; the reference has none.
- * A large product of the tiled family that runs on the bf16 matrix cores (under the AUTO
- * policy, with no tiled tuning override) is described by the fp32 plan it replaces; its own
- * tile and k ranges follow from that plan and the sizes. */
+ * "tiled-split" is a large product of the tiled family that runs on the bf16 matrix cores
+ * (under the AUTO policy, with no tiled tuning override). */
 int migemm_last_plan(char *buf, size_t len);
 
 /* (5) Measurement. Streams src[0 .. n) once -- `blocks` work-groups, each a contiguous

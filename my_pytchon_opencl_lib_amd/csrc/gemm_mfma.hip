@@ -894,12 +894,7 @@ int launch_gemm_tiled(hipStream_t stream, const GemmDesc &d, bool automatic) {
         TiledArgs sa = a;
         sa.write_back = !rows64;
         const int rc = launch_gemm_split(stream, sa, split_plan, akc, bkc);
-        // the record keeps the decomposition it replaces, whose non-empty ranges are
-        const int nk = cfg == 128 && big == 0 ? (d.K + 15) / 16 : nk32;
-        const int per = (nk + std::min(splits, nk) - 1) / std::min(splits, nk);
-        record_plan("tiled-direct", d, cfg == 128 && big == 2 ? 256 : cfg,
-                    cfg == 128 && big >= 1 ? 256 : cfg, (nk + per - 1) / per,
-                    wa == 4 && wb == 4 ? 16 : 4);
+        record_plan("tiled-split", d, split_plan.bm, split_plan.bn, sa.splits, 0);
         if (rc != MIGEMM_OK || sa.splits == 1) return rc;
         return launch_reduce_slices(stream, sa.partial, sa.splits, d.batch, d.M, d.N, d.bias,
                                     d.C, d.ldc, d.sC, d.accumulate);

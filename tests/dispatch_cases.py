@@ -8,6 +8,7 @@ run them and compare the plan a real call records).
             (64 sequences x 100 steps, input 512, hidden 1024): lstm_gemm_xw, lstm_gemm_grad_x,
             the two accumulating weight-gradient GEMMs and one recurrent step;
   AUTO_REGIMES  shapes at the edges of the dispatcher's regimes.
+  FP32      the plans on the fp32 MFMA that the split kernel replaces.
 Each entry is (name, arguments of migemm_gemm_strided_batched_ex as a dict, expected plan).
 Addresses are fixed multiples of 2^32 (the real tests' tensors are at least 512-byte
 aligned, so alignment-dependent choices agree); `off*` shift an operand by elements, as the
@@ -40,13 +41,13 @@ BASELINE = [
     ("cfg3 LSTM gate step + bias", dict(M=64, N=4096, K=1536, bias=True),
      "panel tile=32x32 splits=1 load_bytes=16 M=64 N=4096 K=1536 batch=1 NN"),
     ("cfg4 NN", dict(M=4096, N=4096, K=4096),
-     "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 NN"),
+     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NN"),
     ("cfg4 NT dA", dict(M=4096, N=4096, K=4096, tb=1),
-     "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 NT"),
+     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NT"),
     ("cfg4 TN dB", dict(M=4096, N=4096, K=4096, ta=1),
-     "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 TN"),
+     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 TN"),
     ("cfg5a ragged", dict(M=1000, N=3000, K=777),
-     "tiled-direct tile=64x64 splits=1 load_bytes=4 M=1000 N=3000 K=777 batch=1 NN"),
+     "tiled-split tile=128x128 splits=1 load_bytes=0 M=1000 N=3000 K=777 batch=1 NN"),
     ("cfg5b GEMV", dict(M=1, N=11008, K=4096),
      "skinny tile=0x256 splits=16 load_bytes=0 M=1 N=11008 K=4096 batch=1 NN"),
 ]
@@ -54,25 +55,54 @@ BASELINE = [
 CALLERS = [
     ("Linear forward (C#: W [1, 500, 6565] + bias)",
      dict(M=1500, N=6565, K=500, batch=8, sB=0, bias=True),
-     "tiled-direct tile=128x128 splits=1 load_bytes=4 M=12000 N=6565 K=500 batch=1 NN"),
+     "tiled-split tile=128x128 splits=1 load_bytes=0 M=12000 N=6565 K=500 batch=1 NN"),
     ("Linear forward (Python: W [6565, 500], NT)", dict(M=12000, N=6565, K=500, tb=1),
-     "tiled-direct tile=128x256 splits=1 load_bytes=16 M=12000 N=6565 K=500 batch=1 NT"),
+     "tiled-split tile=128x128 splits=1 load_bytes=0 M=12000 N=6565 K=500 batch=1 NT"),
     ("Linear dX = dY W^T", dict(M=1500, N=500, K=6565, batch=8, tb=1, sB=0),
-     "tiled-direct tile=128x128 splits=4 load_bytes=4 M=12000 N=500 K=6565 batch=1 NT"),
+     "tiled-split tile=256x128 splits=4 load_bytes=0 M=12000 N=500 K=6565 batch=1 NT"),
     ("Linear dW = X^T dY over 12000 rows", dict(M=500, N=6565, K=12000, ta=1),
-     "tiled-direct tile=128x128 splits=6 load_bytes=4 M=500 N=6565 K=12000 batch=1 TN"),
+     "tiled-split tile=128x128 splits=6 load_bytes=0 M=500 N=6565 K=12000 batch=1 TN"),
     ("lstm_gemm_xw", dict(M=6400, N=4096, K=512, bias=True),
-     "tiled-direct tile=64x64 splits=1 load_bytes=16 M=6400 N=4096 K=512 batch=1 NN"),
+     "tiled-split tile=128x128 splits=1 load_bytes=0 M=6400 N=4096 K=512 batch=1 NN"),
     ("lstm_gemm_grad_x", dict(M=6400, N=512, K=4096, tb=1),
-     "tiled-direct tile=64x64 splits=3 load_bytes=16 M=6400 N=512 K=4096 batch=1 NT"),
+     "tiled-split tile=256x256 splits=5 load_bytes=0 M=6400 N=512 K=4096 batch=1 NT"),
     ("lstm grad_W += X^T G", dict(M=512, N=4096, K=6400, ta=1, acc=True),
-     "tiled-direct tile=64x64 splits=1 load_bytes=16 M=512 N=4096 K=6400 batch=1 TN"),
+     "tiled-split tile=128x128 splits=2 load_bytes=0 M=512 N=4096 K=6400 batch=1 TN"),
     ("lstm grad_U += H_prev^T G", dict(M=1024, N=4096, K=6400, ta=1, acc=True),
-     "tiled-direct tile=256x256 splits=4 load_bytes=16 M=1024 N=4096 K=6400 batch=1 TN"),
+     "tiled-split tile=256x256 splits=4 load_bytes=0 M=1024 N=4096 K=6400 batch=1 TN"),
     ("lstm recurrent step t=50", dict(M=64, N=4096, K=1024, acc=True, lda=100 * 1024,
                                       ldc=100 * 4096, offA=49 * 1024, offC=50 * 4096),
      "panel tile=32x32 splits=1 load_bytes=16 M=64 N=4096 K=1024 batch=1 NN"),
 ]
+
+# The plans on the fp32 MFMA that the split kernel replaces (MIGEMM_TUNE_DIRECT = 2 keeps
+# them): name of an entry above -> plan.
+FP32 = {
+    "cfg4 NN":
+        "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 NN",
+    "cfg4 NT dA":
+        "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 NT",
+    "cfg4 TN dB":
+        "tiled-direct tile=256x256 splits=1 load_bytes=16 M=4096 N=4096 K=4096 batch=1 TN",
+    "cfg5a ragged":
+        "tiled-direct tile=64x64 splits=1 load_bytes=4 M=1000 N=3000 K=777 batch=1 NN",
+    "Linear forward (C#: W [1, 500, 6565] + bias)":
+        "tiled-direct tile=128x128 splits=1 load_bytes=4 M=12000 N=6565 K=500 batch=1 NN",
+    "Linear forward (Python: W [6565, 500], NT)":
+        "tiled-direct tile=128x256 splits=1 load_bytes=16 M=12000 N=6565 K=500 batch=1 NT",
+    "Linear dX = dY W^T":
+        "tiled-direct tile=128x128 splits=4 load_bytes=4 M=12000 N=500 K=6565 batch=1 NT",
+    "Linear dW = X^T dY over 12000 rows":
+        "tiled-direct tile=128x128 splits=6 load_bytes=4 M=500 N=6565 K=12000 batch=1 TN",
+    "lstm_gemm_xw":
+        "tiled-direct tile=64x64 splits=1 load_bytes=16 M=6400 N=4096 K=512 batch=1 NN",
+    "lstm_gemm_grad_x":
+        "tiled-direct tile=64x64 splits=3 load_bytes=16 M=6400 N=512 K=4096 batch=1 NT",
+    "lstm grad_W += X^T G":
+        "tiled-direct tile=64x64 splits=1 load_bytes=16 M=512 N=4096 K=6400 batch=1 TN",
+    "lstm grad_U += H_prev^T G":
+        "tiled-direct tile=256x256 splits=4 load_bytes=16 M=1024 N=4096 K=6400 batch=1 TN",
+}
 
 # (spec, expected plan prefix) -- the regime table of the GPU test test_auto_regimes
 AUTO_REGIMES = [
@@ -99,8 +129,8 @@ AUTO_REGIMES = [
     # per lane, >= 6 rounds of tiles): 128x128
     (dict(batch=1, M=8192, K=64, N=8180, ta=0, tb=0), "tiled-direct tile=64x64"),
     (dict(batch=1, M=12592, K=47, N=2304, ta=0, tb=0), "tiled-direct tile=128x128"),
-    # long K over few tiles: 64x64 tiles in k ranges (the LSTM gate gradient)
-    (dict(batch=1, M=6400, K=4096, N=512, ta=0, tb=1), "tiled-direct tile=64x64 splits=3"),
+    # long K over few tiles: k ranges (the LSTM gate gradient)
+    (dict(batch=1, M=6400, K=4096, N=512, ta=0, tb=1), "tiled-split tile=256x256 splits=5"),
     # one row of C, B stored [N, K], few rows: the rows GEMV; 3 rows over a batch whose
     # entries hold small B: the small kernel
     (dict(batch=1, M=1, K=1301, N=440, ta=0, tb=1), "skinny-rows"),

@@ -25,6 +25,13 @@ def test_plan_of_baseline_and_callers(name, spec, plan):
     assert _native.gemm_plan(*dc.args(**spec)) == plan
 
 
+@pytest.mark.parametrize("name", dc.FP32)
+def test_fp32_plan_behind_a_split_one(name):
+    spec = next(s for n, s, _ in dc.BASELINE + dc.CALLERS if n == name)
+    with _native.tuned(direct=2):
+        assert _native.gemm_plan(*dc.args(**spec)) == dc.FP32[name]
+
+
 @pytest.mark.parametrize("spec,plan", dc.AUTO_REGIMES)
 def test_plan_of_regime_table(spec, plan):
     assert _native.gemm_plan(*dc.regime_args(spec)).startswith(plan)
@@ -53,7 +60,9 @@ def test_plan_follows_policy_and_tuning():
         _native.set_gemm_policy(prev)
     with _native.tuned(tile=128, splitk=2):
         assert _native.gemm_plan(*a).startswith("tiled-direct tile=128x128 splits=2 ")
-    assert _native.gemm_plan(*a).startswith("tiled-direct tile=256x256 splits=1 ")
+    with _native.tuned(direct=2):
+        assert _native.gemm_plan(*a).startswith("tiled-direct tile=256x256 splits=1 ")
+    assert _native.gemm_plan(*a).startswith("tiled-split tile=256x256 splits=1 ")
 
 
 # (M, K, N, ta, tb, k ranges of the fp32 plan): products whose split plan has more ranges
@@ -73,9 +82,9 @@ def test_partial_sums_fit_the_workspace_or_another_plan_runs(M, K, N, ta, tb, ra
         with _native.tuned(plan_workspace=kib):
             plan = _native.gemm_plan(*a)
         if kib < 1 << 20:
-            assert f"splits={ranges} " in plan
+            assert plan.startswith("tiled-direct ") and f"splits={ranges} " in plan
         else:
-            assert plan == free
+            assert plan == free and plan.startswith("tiled-split ")
     if ranges > 1:
         with _native.tuned(plan_workspace=fp32 // 1024 - 1):
             with pytest.raises(_native.MigemmRuntimeError, match="bytes of workspace are needed"):

@@ -91,14 +91,14 @@ def test_split_error_no_larger_than_fp32(M, K, N, batch, ta, tb):
     (a, lda, sA), (b, ldb, sB), a64, b64 = case(M, K, N, ta, tb, batch=batch, ints=False, seed=N)
     c64 = a64 @ b64
     err, outs = [], []
-    for direct in (0, 2):  # the dispatcher's choice, then the fp32 kernels
+    for direct, kernel in ((0, "tiled-split "), (2, "tiled-direct ")):
         c = torch.full((batch, M, N), float("nan"), device="cuda:0")
         with _native.tuned(direct=direct):
             run(ta, tb, M, N, K, a, lda, sA, b, ldb, sB, None, c, N, M * N, batch)
+        assert _native.last_plan().startswith(kernel), _native.last_plan()
         err.append(float((c - c64).norm() / c64.norm()))
         outs.append(c)
     say("split error", M, K, N, batch, ta, tb, err)
-    assert not torch.equal(outs[0], outs[1]), "the call did not take the split kernel"
     assert err[0] <= 1.02 * err[1]
 
 
@@ -181,7 +181,8 @@ def test_split_graph_capture_in_a_workspace_for_fewer_ranges():
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=cap):
         run(0, 1, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
-    assert "splits=3 " in _native.last_plan()
+    plan = _native.last_plan()
+    assert plan.startswith("tiled-direct ") and "splits=3 " in plan, plan
     say("replay in 3 ranges")
     for _ in range(3):
         c.fill_(float("nan"))
