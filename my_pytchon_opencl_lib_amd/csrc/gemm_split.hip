@@ -79,11 +79,11 @@ double split_rounds(const SplitFit &f, double t) {
 
 SplitPlan plan_split(const GemmDesc &d, int plan_splits) {
     SplitPlan best = {0, 0, 1, 1e300};
-    // A k-long sum's error grows as the root of its k range and is 0.88-0.95 of the fp32
-    // MFMA's here, so no fewer than 0.77 of the fp32 plan's ranges keep it no larger: the LSTM
-    // input gradient 6400 x 4096 x 512 (3 ranges in fp32, 6.6e-7) has 1.0e-6 in one range,
-    // 5.8e-7 in three.
-    const int least = (77 * plan_splits + 99) / 100;
+    // A k-long sum's error grows as the root of its k range and is 0.83-0.91 of the fp32
+    // MFMA's here, so no fewer ranges than the fp32 plan has keep it no larger: the LSTM input
+    // gradient 6400 x 4096 x 512 (3 ranges in fp32, 6.6e-7) has 1.0e-6 in one range, 5.8e-7 in
+    // three.
+    const int least = plan_splits;
     const int most = plan_splits > 8 ? plan_splits : 8;
     const int nk = (d.K + SBK - 1) / SBK;
     const bool odd = d.ldc % 16 != 0 || ((uintptr_t)d.C & 63) != 0 ||

@@ -5,6 +5,7 @@ regime table (tests/dispatch_cases.py). A change to the dispatcher shows up here
 changed plan string; the GPU suite checks that real calls record the same plans
 (tests/test_gemm_gpu.py::test_dry_run_plans_match_real_calls)."""
 import random
+import re
 
 import pytest
 
@@ -89,6 +90,24 @@ def test_partial_sums_fit_the_workspace_or_another_plan_runs(M, K, N, ta, tb, ra
         with _native.tuned(plan_workspace=fp32 // 1024 - 1):
             with pytest.raises(_native.MigemmRuntimeError, match="bytes of workspace are needed"):
                 _native.gemm_plan(*a)
+
+
+def test_split_plan_has_no_fewer_k_ranges_than_the_fp32_plan():
+    """The error of a sum grows with the root of its k range: over products of 200-13000 the
+    split kernel never runs fewer ranges than the fp32 plan it replaces."""
+    rng = random.Random(3)
+    splits = 0
+    for _ in range(3000):
+        M, K, N = (int(200 * 65 ** rng.random()) // 32 * 32 + rng.choice([0, 5]) for _ in range(3))
+        a = dc.args(M, N, K, ta=rng.randrange(2), tb=rng.randrange(2))
+        plan = _native.gemm_plan(*a)
+        if plan.startswith("tiled-split "):
+            splits += 1
+            with _native.tuned(direct=2):
+                fp32 = _native.gemm_plan(*a)
+            ranges = [int(re.search(r"splits=(\d+) ", p)[1]) for p in (plan, fp32)]
+            assert ranges[0] >= ranges[1], (plan, fp32)
+    assert splits > 500
 
 
 def test_no_plan_launches_k_ranges_without_a_buffer():
