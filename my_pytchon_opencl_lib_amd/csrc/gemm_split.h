@@ -20,8 +20,11 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int SBK = 16;  // k per k-tile: one 32x32x16 MFMA step
 
-// 2 |x| - 1 as bits for |x| = 2^-110; a zero wraps around to the largest value.
-constexpr uint32_t kSplitLeast = 2u * ((127u - 110u) << 23) - 1u;
+// Operand values are scaled by 2^23 before they are split, and the sums by 2^-46 after the k
+// loop, both exact: a multiple of fp32's least subnormal 2^-149 becomes one of 2^-126, so that
+// every part of every value is a normal bf16 number or zero.
+constexpr float kSplitScale = 0x1p+23f;
+constexpr float kSplitUnscale = 0x1p-46f;
 
 template <typename F, int... I>
 __device__ __forceinline__ void unroll_impl(F f, std::integer_sequence<int, I...>) {
@@ -63,12 +66,10 @@ struct SplitOperand {
     uint32_t voff;       // this lane's byte offset from `base` at k-tile 0
     int row;             // row of the tile this thread holds
     int k0;              // its first k of the k-tile
-    uint32_t least;      // least nonzero magnitude seen: min over x of 2 |x| - 1 as bits
 
     __device__ __forceinline__ void init(const float *op, int64_t ld_, int i0, int extent,
                                          int tid) {
         ld = ld_;
-        least = 0xffffffffu;
         base = reinterpret_cast<const char *>(op + (KC ? (int64_t)i0 * ld : (int64_t)i0));
         row = KC ? tid / LPR : tid % T;
         k0 = E * (KC ? tid % LPR : tid / T);
@@ -96,37 +97,39 @@ struct SplitOperand {
         for (int k = 0; k < E; ++k) v[k] = k0 + k >= dup ? v[k] : 0.f;
     }
 
-    // Whether every value put so far splits exactly.
-    __device__ __forceinline__ bool exact() const { return least >= kSplitLeast; }
-
     // Splitting and storing the k-tile in STEPS steps, two for each pair of values: a value x
-    // becomes high + mid + low, each a bf16 rounded to nearest, which is x bit for bit when x
-    // is 0 or at least 2^-110 in magnitude (24 significand bits in three of 8 bits, the lowest
-    // no smaller than bf16's least subnormal 2^-133) and below bf16's rounding overflow
-    // (3.39e38). The first step also notes the least nonzero magnitude. The last one stores
-    // the three parts into `stage`. As volatile assembly the steps stay where the k loop
-    // places them, between MFMAs; as ordinary code the compiler gathers them in one stretch
-    // under no MFMA.
+    // becomes high + mid + low, each a bf16 rounded to nearest, which is x (scaled) bit for bit
+    // below bf16's rounding overflow (|x| < 4.04e31): 24 significand bits in three of 8 bits.
+    // The last step stores the three parts into `stage`. As volatile assembly the steps stay
+    // where the k loop places them, between MFMAs; as ordinary code the compiler gathers them
+    // in one stretch under no MFMA. A step scales one value of the next pair: scaled in the
+    // step that splits them, they lengthen its chain (4096^3 NN / NT / TN 616 / 624 / 624 us,
+    // this way 603 / 597 / 606).
     static constexpr int STEPS = E;
     typedef uint32_t Part __attribute__((ext_vector_type(E / 2)));
     Part h, m, l;
+    static __device__ __forceinline__ void scale(float &x) {
+        asm volatile("v_mul_f32 %0, %1, %0" : "+v"(x) : "s"(kSplitScale));
+    }
     template <int S>
     __device__ __forceinline__ void split_step(uint32_t *stage) {
         constexpr int q = S / 2;
         uint32_t t0, t1;
         if constexpr (S % 2 == 0) {
             uint32_t a;
+            if constexpr (S == 0) {
+                scale(v[0]);
+                scale(v[1]);
+            }
             asm volatile(
-                "v_lshl_add_u32 %[t0], %[x0], 1, -1\n\t"
-                "v_lshl_add_u32 %[t1], %[x1], 1, -1\n\t"
                 "v_cvt_pk_bf16_f32 %[a], %[x0], %[x1]\n\t"
-                "v_min3_u32 %[least], %[least], %[t0], %[t1]\n\t"
                 "v_lshlrev_b32 %[t0], 16, %[a]\n\t"
                 "v_and_b32 %[t1], 0xffff0000, %[a]\n\t"
                 "v_sub_f32 %[x0], %[x0], %[t0]\n\t"
                 "v_sub_f32 %[x1], %[x1], %[t1]"
                 : [a] "=&v"(a), [t0] "=&v"(t0), [t1] "=&v"(t1), [x0] "+v"(v[2 * q]),
-                  [x1] "+v"(v[2 * q + 1]), [least] "+v"(least));
+                  [x1] "+v"(v[2 * q + 1]));
+            if constexpr (S + 2 < STEPS) scale(v[2 * q + 2]);
             h[q] = a;
         } else {
             uint32_t b, c;
@@ -139,6 +142,7 @@ struct SplitOperand {
                 "v_cvt_pk_bf16_f32 %[c], %[x0], %[x1]"
                 : [b] "=&v"(b), [c] "=&v"(c), [t0] "=&v"(t0), [t1] "=&v"(t1),
                   [x0] "+v"(v[2 * q]), [x1] "+v"(v[2 * q + 1]));
+            if constexpr (S + 1 < STEPS) scale(v[2 * q + 3]);
             m[q] = b;
             l[q] = c;
         }
@@ -299,17 +303,19 @@ gemm_split_kernel(TiledArgs p) {
         if (kt + 1 < kt1) step(kt + 1, std::integral_constant<int, 1>{});
     }
 
-    // An operand value that does not split exactly, or an output that is not finite (an
-    // infinity or NaN among the operands, which the parts do not carry, or an overflow): the
-    // tile again in fp32, on the fp32 MFMA.
-    bool bad = !opa.exact() || !opb.exact();
+    // An output that is not finite (an infinity, NaN or value of 4.04e31 or more among the
+    // operands, which the parts do not carry, or a sum of 4.83e24 or more, which overflows
+    // scaled): the tile again in fp32, on the fp32 MFMA.
+    bool bad = false;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
+            for (int r = 0; r < 16; ++r) {
                 bad |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
+                acc[i][j][r] *= kSplitUnscale;
+            }
     if (bad) lds_flag = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(lds_flag) != 0) {

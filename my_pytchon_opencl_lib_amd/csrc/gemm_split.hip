@@ -4,8 +4,7 @@
 // What bounds a large product on the fp32 MFMA is its rate: 157.3 TFLOP/s, of which
 // gemm_direct_kernel reaches 94-95 % at 4096^3. The bf16 MFMA is 16 times as fast, and an
 // fp32 value is the sum of three bf16 values, x = h + m + l (8 significand bits each, rounded
-// to nearest, so the next part carries the signed remainder; bit for bit equal to x from
-// 2^-110 up). Six of the nine products of the parts are computed, the smallest first, into
+// to nearest, so the next part carries the signed remainder; bit for bit equal to x). Six of the nine products of the parts are computed, the smallest first, into
 // one fp32 accumulator per output:
 //   a b = ah bl + al bh + am bm + am bh + ah bm + ah bh;
 // the three left out (am bl, al bm, al bl) are below 2^-26 of |a b|, a quarter of the
@@ -17,7 +16,7 @@
 //
 // The kernel:
 //  * A k-tile of 16 goes global memory -> registers -> split -> LDS once per work-group, so
-//    the split's 14 vector instructions per pair of values are shared by every wavefront that
+//    the split's 13 vector instructions per pair of values are shared by every wavefront that
 //    reads the tile. Its steps run between the MFMAs of the k-tile before (one step of 6-8
 //    instructions behind an MFMA), and the loads of the k-tile after are issued as soon as
 //    the registers are free. Two LDS stages, one barrier per k-tile.
@@ -27,11 +26,15 @@
 //    adjacent rows, for an I-contiguous one; neither needs alignment, so odd leading
 //    dimensions and sizes run the same code. The last k-tile of K % 16 != 0 is read from
 //    k = K - 16 on with the shared k cleared.
-//  * Values the parts cannot carry: a nonzero value below 2^-110 is noticed while splitting;
-//    an infinity, a NaN or a value above 3.39e38 leaves its outputs not finite. A work-group
-//    that meets either computes its tile once more with v_mfma_f32_32x32x2_f32, so infinities,
-//    NaN and the smallest values give what the fp32 kernels give (such a tile costs about
-//    2.5 times an ordinary one).
+//  * Operand values are scaled by 2^23 while they are split and the sums by 2^-46 at the end:
+//    the parts of every fp32 value, subnormal ones too, are then normal bf16 numbers, and no
+//    tile is computed in another way for its small values (4096^3 with one value of 1e-35 in
+//    every row of A, us: tiles with values below 2^-110 a second time in fp32 1698, so 601;
+//    without such values 619 and 599).
+//  * Values the parts cannot carry: an infinity, a NaN or a value of 4.04e31 or more leaves
+//    its outputs not finite, and so does a sum of 4.83e24 or more. A work-group that meets one
+//    computes its tile once more with v_mfma_f32_32x32x2_f32, so these give what the fp32
+//    kernels give (such a tile costs about 2.5 times an ordinary one).
 //
 // Measured (events around 10 launches, N(0,1) operands, us, this kernel / the fp32 choice):
 // 4096^3 NN 650 / 910, NT 605 / 908, TN 610 / 906 (211-227 TFLOP/s); 12000 x 500 x 6565

@@ -104,9 +104,9 @@ def test_split_error_no_larger_than_fp32(M, K, N, batch, ta, tb):
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
 def test_split_nonfinite_and_tiny_operands(ta, tb):
-    """Infinities and NaN reach the outputs that fp32 arithmetic says, values below 2^-110
-    keep their precision, a value above bf16's rounding overflow stays finite, and every
-    other output is the exact product."""
+    """Infinities and NaN reach the outputs that fp32 arithmetic says, tiny values keep their
+    precision, a value above bf16's rounding overflow stays finite, and every other output is
+    the exact product."""
     M, K, N = 2100, 1009, 1900
     (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, seed=5)
 
@@ -131,7 +131,11 @@ def test_split_nonfinite_and_tiny_operands(ta, tb):
     assert torch.equal(torch.nan_to_num(got[rows], nan=123.5), torch.nan_to_num(expect[rows], nan=123.5))
     big = got[1900, :1899].double() / expect[1900, :1899].double()
     assert bool(((big - 1).abs() < 1e-6).all())
-    # tiny: A of 2^-126 .. 2^-122, B scaled up by 2^60
+    # sums past 2^82, which overflow scaled, stay finite too (here |sum| <= 16 K 2^110 < 2^124)
+    (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, seed=7)
+    run(ta, tb, M, N, K, a * 2.0 ** 55, lda, 0, b * 2.0 ** 55, ldb, 0, None, c, N, 0)
+    assert torch.equal(c, (a64 @ b64)[0].float() * 2.0 ** 110)
+    # tiny: A of 2^-126 .. 2^-122, subnormals among them, B scaled up by 2^60
     (a, lda, _), (b, ldb, _), a64, b64 = case(M, K, N, ta, tb, ints=False, seed=6)
     a *= 2.0 ** -124
     b *= 2.0 ** 60
@@ -140,6 +144,38 @@ def test_split_nonfinite_and_tiny_operands(ta, tb):
     run(ta, tb, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
     c64 = a64 @ b64
     assert float((c.double() - c64).norm() / c64.norm()) < 1e-6  # fp32 chain: 5.7e-7
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+def test_split_small_operands_bit_for_bit(ta, tb):
+    """A power of two times an operand is that power times the result, bit for bit, down to
+    fp32's least normal and subnormal values (every bf16 part of a scaled value is a normal
+    number): no precision is lost on the way and no tile is computed in another way, whose
+    bits would differ."""
+    M, K, N = 2100, 1009, 1900
+    (a, lda, _), (b, ldb, _), _, _ = case(M, K, N, ta, tb, ints=False, seed=21)
+    a.copy_((1 + a.abs() % 15) * a.sign())  # magnitudes of [1, 16): normal down to 2^-126
+    b.copy_((1 + b.abs() % 15) * b.sign())
+
+    def product(x, y):
+        c = torch.full((M, N), float("nan"), device="cuda:0")
+        run(ta, tb, M, N, K, x, lda, 0, y, ldb, 0, None, c, N, 0)
+        assert _native.last_plan().startswith("tiled-split "), _native.last_plan()
+        return c
+
+    plain = product(a, b)
+    for e in (60, 103, 110, 126):
+        say("split small operands", ta, tb, e)
+        small = 2.0 ** -(e // 2) * 2.0 ** -(e - e // 2)
+        assert torch.equal(product(a * small, b * 2.0 ** 40) * 2.0 ** (e - 40), plain)
+        assert torch.equal(product(a * 2.0 ** 40, b * small) * 2.0 ** (e - 40), plain)
+    # n 2^-149 for integers |n| < 2^23 are the floats whose bits are n
+    g = torch.Generator(device="cuda:0").manual_seed(22)
+    n = torch.randint(1, 1 << 23, a.shape, generator=g, device="cuda:0", dtype=torch.int32)
+    sign = torch.where(a < 0, -1.0, 1.0)
+    tiny = torch.copysign(n.view(torch.float32), sign)
+    c = product(tiny, b * 2.0 ** 100)
+    assert torch.equal(c * 2.0 ** 49, product(n.float() * sign, b))
 
 
 def test_split_graph_capture_without_a_workspace():
