@@ -316,7 +316,7 @@ def main():
     cpu = None if args.no_cpu_baseline else cpu_baseline(args.cpu_seconds)
 
     prof = load_profiled(SPLIT_TRACE_SUMMARY)
-    roofline = {"bound": "mfma", "kernel": f"gemm_split_kernel ({dominant} form, 256x256 tiles)",
+    roofline = {"bound": "mfma", "kernel": f"gemm_split_kernel ({dominant} form, 256x128 tiles)",
                 "achieved": round(achieved, 3), "peak": PEAK_SPLIT_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / PEAK_SPLIT_TFLOPS, 4),
                 "peak_is": "dense bf16 MFMA rate / 6 (bf16 products per fp32 product)",
@@ -480,7 +480,7 @@ def summarize_trace(directory, steps, warmup):
         short = short.replace("void ", "")
         us = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
         by_kernel.setdefault(short, []).append(us)
-        m = re.search(r"gemm_(?:direct|split)_kernel<256, 256, \d+, \d+, "
+        m = re.search(r"gemm_(?:direct_kernel<256, 256|split_kernel<256, 128), \d+, \d+, "
                       r"(true|false), (true|false)", name)
         if m:
             forms.setdefault(FORM_OF[m.groups()], []).append(us)

@@ -10,7 +10,6 @@
 namespace migemm {
 
 // Per tile shape: launches gemm_split_kernel for the operand layouts (akc, bkc).
-int launch_split_256(hipStream_t stream, TiledArgs &a, bool akc, bool bkc);
 int launch_split_256x128(hipStream_t stream, TiledArgs &a, bool akc, bool bkc);
 int launch_split_128(hipStream_t stream, TiledArgs &a, bool akc, bool bkc);
 
@@ -165,7 +164,8 @@ struct SplitOperand {
 };
 
 template <int BM, int BN, int WM, int WN, bool AKC, bool BKC>
-__global__ void __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(WM *WN * 64)
+    __attribute__((amdgpu_waves_per_eu(BM * BN <= 128 * 128 ? 4 : 2)))  // work-groups per CU: 2, 1
 gemm_split_kernel(TiledArgs p) {
     constexpr int NT = WM * WN * 64;
     constexpr int WTM = BM / WM;
@@ -200,14 +200,14 @@ gemm_split_kernel(TiledArgs p) {
     opa.init(p.A + (int64_t)tc.b * p.sA, p.lda, tc.m0, p.M, tid);
     opb.init(p.B + (int64_t)tc.b * p.sB, p.ldb, tc.n0, p.N, tid);
 
-    f16 acc[FM][FN];
+    f16 acc[FM][FN], low[FM][FN];  // sums of the high parts' products, of the others
     auto clear = [&]() {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.f;
     };
     clear();
     if (tid == 0) lds_flag = 0;
@@ -239,8 +239,8 @@ gemm_split_kernel(TiledArgs p) {
         }
     };
 
-    // The products of two parts (0 high, 1 mid, 2 low), the smallest first; the three that
-    // are left out are below 2^-26 of the product.
+    // The products of two parts (0 high, 1 mid, 2 low), the smallest first (gemm_split.hip: what
+    // the three that are left out amount to, and why the last has a sum of its own).
     constexpr int PA[6] = {0, 2, 1, 1, 0, 0};
     constexpr int PB[6] = {2, 0, 1, 0, 1, 0};
     bf8 fa[3][FM], fb[3][2];
@@ -277,10 +277,10 @@ gemm_split_kernel(TiledArgs p) {
             constexpr int j0 = N / (12 * FM) * 2, q = N / (2 * FM) % 6;
             constexpr int i = N / 2 % FM, j = N % 2;
             __builtin_amdgcn_sched_barrier(0);
-            acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                fa[PA[q]][i], fb[PB[q]][j], acc[i][j0 + j], 0, 0, 0);
+            f16 &c = q == 5 ? acc[i][j0 + j] : low[i][j0 + j];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[PA[q]][i], fb[PB[q]][j], c, 0, 0, 0);
             // (an MFMA has no side effect: without a use here it is moved down)
-            asm volatile("" : "+v"(acc[i][j0 + j]));
+            asm volatile("" : "+v"(c));
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (i == FM - 1 && j == 1 && j0 + 2 < FN) {
                 if constexpr (q == 0) read_b(ST, j0 + 2, 2);
@@ -313,6 +313,7 @@ gemm_split_kernel(TiledArgs p) {
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] += low[i][j][r];
                 bad |= !(__builtin_fabsf(acc[i][j][r]) < __builtin_inff());
                 acc[i][j][r] *= kSplitUnscale;
             }

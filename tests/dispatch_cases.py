@@ -41,11 +41,11 @@ BASELINE = [
     ("cfg3 LSTM gate step + bias", dict(M=64, N=4096, K=1536, bias=True),
      "panel tile=32x32 splits=1 load_bytes=16 M=64 N=4096 K=1536 batch=1 NN"),
     ("cfg4 NN", dict(M=4096, N=4096, K=4096),
-     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NN"),
+     "tiled-split tile=256x128 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NN"),
     ("cfg4 NT dA", dict(M=4096, N=4096, K=4096, tb=1),
-     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NT"),
+     "tiled-split tile=256x128 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 NT"),
     ("cfg4 TN dB", dict(M=4096, N=4096, K=4096, ta=1),
-     "tiled-split tile=256x256 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 TN"),
+     "tiled-split tile=256x128 splits=1 load_bytes=0 M=4096 N=4096 K=4096 batch=1 TN"),
     ("cfg5a ragged", dict(M=1000, N=3000, K=777),
      "tiled-split tile=128x128 splits=1 load_bytes=0 M=1000 N=3000 K=777 batch=1 NN"),
     ("cfg5b GEMV", dict(M=1, N=11008, K=4096),
@@ -65,11 +65,11 @@ CALLERS = [
     ("lstm_gemm_xw", dict(M=6400, N=4096, K=512, bias=True),
      "tiled-split tile=128x128 splits=1 load_bytes=0 M=6400 N=4096 K=512 batch=1 NN"),
     ("lstm_gemm_grad_x", dict(M=6400, N=512, K=4096, tb=1),
-     "tiled-split tile=256x256 splits=5 load_bytes=0 M=6400 N=512 K=4096 batch=1 NT"),
+     "tiled-split tile=256x128 splits=5 load_bytes=0 M=6400 N=512 K=4096 batch=1 NT"),
     ("lstm grad_W += X^T G", dict(M=512, N=4096, K=6400, ta=1, acc=True),
      "tiled-split tile=128x128 splits=2 load_bytes=0 M=512 N=4096 K=6400 batch=1 TN"),
     ("lstm grad_U += H_prev^T G", dict(M=1024, N=4096, K=6400, ta=1, acc=True),
-     "tiled-split tile=256x256 splits=4 load_bytes=0 M=1024 N=4096 K=6400 batch=1 TN"),
+     "tiled-split tile=256x128 splits=4 load_bytes=0 M=1024 N=4096 K=6400 batch=1 TN"),
     ("lstm recurrent step t=50", dict(M=64, N=4096, K=1024, acc=True, lda=100 * 1024,
                                       ldc=100 * 4096, offA=49 * 1024, offC=50 * 4096),
      "panel tile=32x32 splits=1 load_bytes=16 M=64 N=4096 K=1024 batch=1 NN"),
@@ -130,7 +130,7 @@ AUTO_REGIMES = [
     (dict(batch=1, M=8192, K=64, N=8180, ta=0, tb=0), "tiled-direct tile=64x64"),
     (dict(batch=1, M=12592, K=47, N=2304, ta=0, tb=0), "tiled-direct tile=128x128"),
     # long K over few tiles: k ranges (the LSTM gate gradient)
-    (dict(batch=1, M=6400, K=4096, N=512, ta=0, tb=1), "tiled-split tile=256x256 splits=5"),
+    (dict(batch=1, M=6400, K=4096, N=512, ta=0, tb=1), "tiled-split tile=256x128 splits=5"),
     # one row of C, B stored [N, K], few rows: the rows GEMV; 3 rows over a batch whose
     # entries hold small B: the small kernel
     (dict(batch=1, M=1, K=1301, N=440, ta=0, tb=1), "skinny-rows"),

@@ -63,7 +63,7 @@ def test_plan_follows_policy_and_tuning():
         assert _native.gemm_plan(*a).startswith("tiled-direct tile=128x128 splits=2 ")
     with _native.tuned(direct=2):
         assert _native.gemm_plan(*a).startswith("tiled-direct tile=256x256 splits=1 ")
-    assert _native.gemm_plan(*a).startswith("tiled-split tile=256x256 splits=1 ")
+    assert _native.gemm_plan(*a).startswith("tiled-split tile=256x128 splits=1 ")
 
 
 # (M, K, N, ta, tb, k ranges of the fp32 plan): products whose split plan has more ranges

@@ -1,7 +1,7 @@
 """GPU tests of gemm_split_kernel: large products on the bf16 matrix cores, every operand
 value split into three bf16 parts (gemm_split.hip), taken by the dispatcher's own choice.
 
-The shapes reach its three tiles (256x256, 256x128, 128x128), ragged M and N, k-tiles of 16
+The shapes reach its two tiles (256x128, 128x128), ragged M and N, k-tiles of 16
 with every kind of tail, and k ranges. Small-integer operands make the exact answer known in
 any summation order. On random operands the error against fp64 is compared with that of the
 fp32 kernels on the same call (direct loads forced: no split), which it must not exceed, and
@@ -51,7 +51,7 @@ def case(M, K, N, ta, tb, batch=1, pad=0, off=0, ints=True, seed=0):
     return (a, lda, sA), (b, ldb, sB), a64, b64
 
 
-# 128x128 (2100 x 1009 x 1900), 256x128 and 256x256 tiles; K % 16 = 0, 1, 15 and 9
+# 128x128 and 256x128 (3073 x 2048 x 4225) tiles; K % 16 = 0, 1 and 15
 SHAPES = [(2100, 1009, 1900), (4097, 144, 3073), (5000, 511, 2049), (3073, 2048, 4225)]
 
 
@@ -100,6 +100,73 @@ def test_split_error_no_larger_than_fp32(M, K, N, batch, ta, tb):
         outs.append(c)
     say("split error", M, K, N, batch, ta, tb, err)
     assert err[0] <= 1.02 * err[1]
+
+
+# Operands of real use that are not dense: (name, A of N(0,1) values -> A)
+SPARSE = [("relu", lambda a, g: a.clamp(min=0)),
+          ("quarter", lambda a, g: a * (torch.rand(a.shape, generator=g, device=a.device) < 0.25)),
+          ("sixteen in K", lambda a, g: a * (torch.rand(a.shape, generator=g, device=a.device)
+                                             < 16.0 / 1009)),
+          ("positive", lambda a, g: a.abs())]
+
+
+@pytest.mark.parametrize("name,change", SPARSE, ids=[s[0] for s in SPARSE])
+@pytest.mark.parametrize("M,K,N", [(2100, 1009, 1900), (2500, 4095, 2500), (500, 12000, 6565)])
+def test_split_error_of_sparse_and_one_sided_operands(M, K, N, name, change):
+    """As above for operands with zeros, around which each rounding of a sum tells, and for
+    values of one sign, whose sums show a rounding that is not to nearest."""
+    (a, lda, _), (b, ldb, _), _, b64 = case(M, K, N, 0, 0, ints=False, seed=K)
+    g = torch.Generator(device="cuda:0").manual_seed(31)
+    a = change(a, g).contiguous()
+    if name == "positive":
+        b = b.abs()
+    c64 = a.view(M, K).double() @ b.view(K, N).double()
+    err = []
+    for direct, kernel in ((0, "tiled-split "), (2, "tiled-direct ")):
+        c = torch.full((M, N), float("nan"), device="cuda:0")
+        with _native.tuned(direct=direct):
+            run(0, 0, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+        assert _native.last_plan().startswith(kernel), _native.last_plan()
+        err.append(float((c - c64).norm() / c64.norm()))
+    say("split error", name, M, K, N, err)
+    assert err[0] <= err[1]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+def test_split_sums_of_one_product(ta, tb):
+    """One value per row of op(A): each output is one product, whose error has no sum to hide
+    in. The bound: the products of parts that are left out, (1 + 2^-10) 2^-24 of it; the fp32
+    rounding of the result, 2^-24; five roundings or truncations of a sum below 2^-6 of it,
+    under 2^-27 together. Values near 1 are the worst. Integer products of up to 24 bits are
+    exact."""
+    M, K, N = 2100, 1009, 1900
+    (a, lda, _), (b, ldb, _), _, _ = case(M, K, N, ta, tb, ints=False, seed=41)
+    g = torch.Generator(device="cuda:0").manual_seed(42)
+    at = torch.randint(K, (M,), generator=g, device="cuda:0")
+    m = torch.arange(M, device="cuda:0")
+
+    def product(av, bv):  # values of the M entries and of op(B)
+        a.zero_()
+        a.view(*((K, M) if ta else (M, K)))[(at, m) if ta else (m, at)] = av
+        b.copy_((bv.t() if tb else bv).reshape(-1))
+        c = torch.full((M, N), float("nan"), device="cuda:0")
+        run(ta, tb, M, N, K, a, lda, 0, b, ldb, 0, None, c, N, 0)
+        assert _native.last_plan().startswith("tiled-split "), _native.last_plan()
+        return c.double(), av.double()[:, None] * bv.double()[at]
+
+    uniform = lambda *s: torch.rand(*s, generator=g, device="cuda:0")  # noqa: E731
+    worst = []
+    for av, bv in [(1 + 0.05 * uniform(M), 1 + 0.05 * uniform(K, N)),
+                   (uniform(M) - 0.5, uniform(K, N) - 0.5)]:
+        c, expect = product(av, bv)
+        worst.append(float(((c - expect).abs() / expect.abs().clamp(min=1e-30)).max()) * 2 ** 24)
+    say("split one product", ta, tb, worst)
+    assert max(worst) <= 2.13
+    for bits in (12, 17):  # 12 x 12 and 17 x 7 bits
+        c, expect = product(
+            torch.randint(1 << bits, (M,), generator=g, device="cuda:0").float(),
+            torch.randint(1 << (24 - bits), (K, N), generator=g, device="cuda:0").float())
+        assert torch.equal(c, expect)
 
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
