@@ -51,25 +51,48 @@ def case(M, K, N, ta, tb, batch=1, pad=0, off=0, ints=True, seed=0):
     return (a, lda, sA), (b, ldb, sB), a64, b64
 
 
-# 128x128 and 256x128 (3073 x 2048 x 4225) tiles; K % 16 = 0, 1 and 15
-SHAPES = [(2100, 1009, 1900), (4097, 144, 3073), (5000, 511, 2049), (3073, 2048, 4225)]
+# (M, K, N, tile, k ranges): both tiles, whole and in ranges; K % 16 = 1, 0, 15, 9, 15, 11
+SHAPES = [(2100, 1009, 1900, "128x128", 1), (4097, 144, 3073, "128x128", 1),
+          (5000, 511, 2049, "128x128", 1), (3552, 1865, 2240, "256x128", 1),
+          (2144, 2495, 1024, "256x128", 3), (1030, 2571, 1290, "128x128", 2)]
 
 
-@pytest.mark.parametrize("M,K,N", SHAPES)
+def wide_ints(shape, bits, nonzero, g):
+    """Integers of `bits` bits, `nonzero` of them in each row and the others 0."""
+    keep = torch.rand(shape, generator=g, device="cuda:0").argsort(-1) < nonzero
+    return torch.randint(1 - (1 << bits), 1 << bits, shape, generator=g,
+                         device="cuda:0").float() * keep
+
+
+@pytest.mark.parametrize("M,K,N,tile,ranges", SHAPES)
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
-def test_split_exact(M, K, N, ta, tb):
-    """Odd sizes, rows off 16-byte boundaries, NaN between the rows; bias and C += result."""
-    for pad, off, bias, acc in [(0, 0, False, False), (3, 1, True, True)]:
-        say("split exact", M, K, N, ta, tb, pad, off, bias, acc)
+def test_split_exact(M, K, N, tile, ranges, ta, tb):
+    """Odd sizes, rows off 16-byte boundaries, NaN between the rows; bias and C += result.
+    One operand's integers have mid and low parts too: of 18 bits, 16 to a sum, the other
+    one's of up to 3 (|sum| <= 16 2^18 4 = 2^24)."""
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    for pad, off, bias, acc, wide in [(0, 0, False, False, "a"), (3, 1, True, True, "b"),
+                                      (0, 0, False, False, "")]:
+        say("split exact", M, K, N, ta, tb, pad, off, bias, acc, wide)
         (a, lda, sA), (b, ldb, sB), a64, b64 = case(M, K, N, ta, tb, pad=pad, off=off, seed=K)
+        if wide == "a":
+            a64 = wide_ints((M, K), 18, 16, g).double()[None]
+            a.view(-1, lda)[:, :lda - pad] = a64[0].t() if ta else a64[0]
+        elif wide == "b":
+            b64 = wide_ints((N, K), 18, 16, g).double().t()[None].contiguous()
+            b.view(-1, ldb)[:, :ldb - pad] = b64[0].t() if tb else b64[0]
+        # (with bias and C too, the sums stay below 2^24: checked)
         bv = torch.arange(N, device="cuda:0").remainder(41).sub(20).float() if bias else None
         c = torch.full((M, N + pad), 7.0 if acc else float("nan"), device="cuda:0")
         run(ta, tb, M, N, K, a, lda, sA, b, ldb, sB, bv, c, N + pad, 0, acc=acc)
+        plan = _native.last_plan()
+        assert plan.startswith(f"tiled-split tile={tile} splits={ranges} "), plan
         expect = (a64 @ b64)[0]
         if bias:
             expect = expect + bv.double()
         if acc:
             expect = expect + 7.0
+        assert float(expect.abs().max()) < 2 ** 24
         assert torch.equal(c[:, :N], expect.float())
         if pad:
             assert bool((c[:, N:] == 7.0).all() if acc else c[:, N:].isnan().all())
