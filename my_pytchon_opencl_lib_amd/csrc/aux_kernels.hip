@@ -95,6 +95,9 @@ struct TransposeArgs {
     uint64_t rstride[MAXD], ostride[MAXD];
 };
 
+// Work-groups of 256 threads that one launch can hold: a grid has fewer than 2^32 threads.
+constexpr int64_t kMaxGroups = ((int64_t)1 << 24) - 1;
+
 constexpr int TR = 64;        // tile edge
 constexpr int TR_GROUP = 32;  // tiles of r rastered together
 
@@ -438,7 +441,7 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
     const int64_t outer = total / behind;
     const int64_t tiles_r = (R + TR - 1) / TR, tiles_c = (cd[jc] + TR - 1) / TR;
     if (jc < nd - 1 && (jc == 0 || behind >= 1024) && R <= INT32_MAX && cd[jc] <= INT32_MAX &&
-        outer * tiles_r * tiles_c <= INT32_MAX && TR_GROUP * tiles_c <= INT32_MAX) {
+        outer * tiles_r * tiles_c <= kMaxGroups && TR_GROUP * tiles_c <= INT32_MAX) {
         TransposeArgs a;
         a.src = src;
         a.dst = dst;

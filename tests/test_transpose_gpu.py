@@ -35,3 +35,19 @@ def test_kernel_choice(nncl, shape, axes, kernel):
     x = torch.randn(shape, device="cuda:0")
     assert torch.equal(nncl.Permute(x, axes), x.permute(axes).contiguous())
     assert _native.last_plan().startswith(kernel + " "), _native.last_plan()
+
+
+@pytest.mark.parametrize("outer,kernel", [((1 << 21) - 1, "transpose"),
+                                          (1 << 21, "permute_gather")])
+def test_more_tiles_than_one_launch_holds(nncl, outer, kernel):
+    """2 x 512 elements per batch entry are 8 tiles: 2^21 entries would need 2^24 work-groups of
+    256 threads, one more than a grid holds, and run through the gather kernel."""
+    print("tiles of one launch", outer, flush=True)
+    x = torch.randn(1 << 20, device="cuda:0").repeat(outer // 1024 + 1)[:outer * 1024]
+    x = x.view(outer, 2, 512)
+    got = nncl.Permute(x, (0, 2, 1))
+    assert _native.last_plan().startswith(kernel + " "), _native.last_plan()
+    for i in range(0, outer, 1 << 18):
+        assert torch.equal(got[i:i + (1 << 18)], x[i:i + (1 << 18)].transpose(1, 2))
+    del x, got
+    torch.cuda.empty_cache()
