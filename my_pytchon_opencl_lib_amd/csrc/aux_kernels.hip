@@ -71,7 +71,8 @@ __global__ void __launch_bounds__(256) permute_gather_kernel(PermuteArgs a) {
 // A batched transpose is the case of one axis behind c.
 //  * HBM-bound: 64x64 tiles through LDS, 16 bytes per lane on both sides (no alignment
 //    needed), so a row of the tile is 256 contiguous bytes read and 256 written. LDS rows of
-//    65 floats keep the scalar writes and reads on distinct banks.
+//    65 floats keep the scalar writes and reads on distinct banks. Matrices that a tile of
+//    32x32 holds or that fill only half of a 64-wide one take 32x32 tiles (launch_permute).
 //  * Consecutive work-groups of an XCD step along r, in groups of 32 tiles: where dst rows do
 //    not start on 128-byte lines, neighbouring tiles share lines, and L2 merges the two parts
 //    before the line goes to HBM. Whole columns of tiles would touch every page of a large
@@ -98,7 +99,6 @@ struct TransposeArgs {
 // Work-groups of 256 threads that one launch can hold: a grid has fewer than 2^32 threads.
 constexpr int64_t kMaxGroups = ((int64_t)1 << 24) - 1;
 
-constexpr int TR = 64;        // tile edge
 constexpr int TR_GROUP = 32;  // tiles of r rastered together
 
 __device__ __forceinline__ uint64_t unpack_offset(uint32_t t, int n, const FastDiv *div,
@@ -112,6 +112,7 @@ __device__ __forceinline__ uint64_t unpack_offset(uint32_t t, int n, const FastD
     return off + t * stride[n - 1];
 }
 
+template <int TR>  // tile edge
 __global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
     typedef float vec __attribute__((ext_vector_type(4)));
     __shared__ float tile[TR][TR + 1];
@@ -132,14 +133,15 @@ __global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
     const uint32_t r0 = tr * TR;
     const uint32_t c0 = tc * TR;
     const uint64_t obase = a.no > 0 ? unpack_offset(o, a.no, a.odiv, a.ostride) : 0;
-    const uint32_t lane4 = 4 * (threadIdx.x & 15);  // this thread's 4 columns (rows of dst)
-    const uint32_t line = threadIdx.x >> 4;         // and its line of each 16
+    const uint32_t lane4 = 4 * (threadIdx.x % (TR / 4));  // this thread's 4 columns (rows of dst)
+    const uint32_t line = threadIdx.x / (TR / 4);   // and its line of each LINES
     const uint32_t nr = min((uint32_t)TR, a.R - r0), nc = min((uint32_t)TR, a.C - c0);
     const float *s = a.src + obase + c0;
-    vec v[4];
+    constexpr int LINES = 1024 / TR, PASSES = TR / LINES;
+    vec v[PASSES];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t r = line + 16 * j;
+    for (int j = 0; j < PASSES; ++j) {
+        const uint32_t r = line + LINES * j;
         if (r < nr) {
             const float *q = s + unpack_offset(r0 + r, a.nr, a.rdiv, a.rstride) + lane4;
             if (lane4 + 4 <= nc) {
@@ -151,8 +153,8 @@ __global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t r = line + 16 * j;
+    for (int j = 0; j < PASSES; ++j) {
+        const uint32_t r = line + LINES * j;
         if (r < nr)
 #pragma unroll
             for (int e = 0; e < 4; ++e) tile[r][lane4 + e] = v[j][e];
@@ -160,8 +162,8 @@ __global__ void __launch_bounds__(256) transpose_kernel(TransposeArgs a) {
     __syncthreads();
     float *d = a.dst + ((size_t)o * a.C + c0) * a.R + r0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t c = line + 16 * j;
+    for (int j = 0; j < PASSES; ++j) {
+        const uint32_t c = line + LINES * j;
         if (c < nc) {
             vec x;
 #pragma unroll
@@ -428,19 +430,27 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
         cs[0] = 1;
         nd = 1;
     }
-    // The source's contiguous axis is not the innermost destination axis: through LDS tiles,
-    // unless a step of the axes before it holds fewer than 1024 elements, most of a tile then
-    // empty (us, gather / tiles: 64000 x 16 x 16 41.5 / 56.6, 200000 x 4 x 16 28.4 / 147.6,
-    // 20000 x 8 x 100 36.6 / 42.5; 4000 x 16 x 64 14.0 / 9.2, 20000 x 32 x 32 78.4 / 36.3).
+    // The source's contiguous axis (C elements) is not the innermost destination axis: through
+    // LDS tiles where these are full enough. A 64x64 tile takes about 1.0 ns of the chip, a
+    // 32x32 one 0.6, an element of the gather kernel 2.2 ps and up, and the memory 1.3 ps an
+    // element. So the tiles are 32x32 for C <= 32 unless R leaves over a quarter of several
+    // tiles empty (us of 2^24 elements as outer x R x C, 64x64 / 32x32: 24 x 24 35.0 / 24.5, 512
+    // x 32 25.8 / 21.0, 130 x 16 35.3 / 30.4; 40 x 32 23.6 / 26.5, 16 x 130 28.9 / 32.2), and
+    // tiles with fewer than `full` elements are left to the gather kernel (tiles / gather: 8 x 130
+    // 48.6 / 37.4, 16 x 16 43.9 / 41.0, 8388608 x 2 134 / 37, 4194304 x 4 71 / 50; 8 x 64 38.0 /
+    // 37.6, 16 x 20 37.9 / 39.4, 64 x 7 51.4 / 39.4, 64 x 8 44.2 / 42.6, 1000 x 7 40.9 / 61.3,
+    // 2097152 x 8 38 / 84).
     int jc = 0;  // its place
     while (cs[jc] != 1) ++jc;
-    int64_t behind = 1;  // elements per step of the axes before it
-    for (int i = jc; i < nd; ++i) behind *= cd[i];
+    const int64_t C = cd[jc];
     int64_t R = 1;
     for (int i = jc + 1; i < nd; ++i) R *= cd[i];
-    const int64_t outer = total / behind;
-    const int64_t tiles_r = (R + TR - 1) / TR, tiles_c = (cd[jc] + TR - 1) / TR;
-    if (jc < nd - 1 && (jc == 0 || behind >= 1024) && R <= INT32_MAX && cd[jc] <= INT32_MAX &&
+    const int64_t outer = total / (R * C);
+    const bool small = C <= 32 && (R <= 32 || 4 * R >= 3 * 32 * ((R + 31) / 32));
+    const int TR = small ? 32 : 64;
+    const int full = !small ? 512 : R <= 32 ? 320 : R <= 128 ? 256 : 224;
+    const int64_t tiles_r = (R + TR - 1) / TR, tiles_c = (C + TR - 1) / TR;
+    if (jc < nd - 1 && R * C >= full * tiles_r * tiles_c && R <= INT32_MAX && C <= INT32_MAX &&
         outer * tiles_r * tiles_c <= kMaxGroups && TR_GROUP * tiles_c <= INT32_MAX) {
         TransposeArgs a;
         a.src = src;
@@ -455,13 +465,16 @@ int launch_permute(hipStream_t stream, const float *src, float *dst, const int *
             a.ostride[a.no] = (uint64_t)cs[i];
         }
         a.R = (uint32_t)R;
-        a.C = (uint32_t)cd[jc];
+        a.C = (uint32_t)C;
         a.tiles_r = (uint32_t)tiles_r;
         a.in_group = make_fastdiv((uint32_t)(TR_GROUP * tiles_c));
         a.last_group = make_fastdiv((uint32_t)(tiles_r % TR_GROUP));
         a.by_rc = make_fastdiv((uint32_t)(tiles_r * tiles_c));
         a.total = (uint32_t)(outer * tiles_r * tiles_c);
-        MIGEMM_LAUNCH(transpose_kernel, dim3(a.total), dim3(256), 0, stream, a);
+        if (small)
+            MIGEMM_LAUNCH(transpose_kernel<32>, dim3(a.total), dim3(256), 0, stream, a);
+        else
+            MIGEMM_LAUNCH(transpose_kernel<64>, dim3(a.total), dim3(256), 0, stream, a);
         record_plan(PlanRecord{"transpose", TR, TR, 1, 16, (int)a.R, (int)a.C, 0, (int)outer,
                                false, false});
         return launch_status("transpose_kernel launch");
