@@ -523,10 +523,11 @@ int launch_column_sum(hipStream_t stream, const float *X, float *Y, int outer, i
             workspace(stream, (size_t)chunks * outer * inner * sizeof(float), &st));
         if (dst == nullptr) return st;
     }
-    if (inner == 1 && !accumulate && rows == CS_ROWS && outer >= 64 && axis >= 16) {
+    const int64_t blocks = ((int64_t)outer + RS_TILE - 1) / RS_TILE;
+    if (inner == 1 && !accumulate && rows == CS_ROWS && outer >= 64 && axis >= 16 &&
+        blocks <= kMaxGroups) {
         // Rows shorter than 16 stay below: two lanes' worth of a tile. Fewer than 64 rows
         // would leave lanes of every tile idle.
-        const int blocks = (outer + RS_TILE - 1) / RS_TILE;
         // with 512 or more work-groups of rows, or one group of chunks, a work-group takes
         // whole rows
         const bool whole = chunks <= 4 || blocks >= 512;

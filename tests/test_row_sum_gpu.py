@@ -37,3 +37,19 @@ def test_short_or_few_rows_keep_the_column_kernel(nncl):
         t = torch.ones(rows, axis, device="cuda:0")
         assert torch.equal(nncl.Sum(t, 1), torch.full((rows,), float(axis), device="cuda:0"))
         assert _native.last_plan().startswith("column_sum"), _native.last_plan()
+
+
+@pytest.mark.parametrize("rows,kernel", [((1 << 30) - 64, "row_sum"), (1 << 30, "column_sum")])
+def test_more_rows_than_one_launch_holds(nncl, rows, kernel):
+    """row_sum_kernel starts 4 threads per row: 2^30 rows need 2^32, one more than a grid
+    holds, and run through the column kernel (64 GiB of values)."""
+    print("rows of one launch", rows, flush=True)
+    t = torch.empty(rows, 16, device="cuda:0")
+    t.copy_(torch.arange(16.0, device="cuda:0"))
+    t[rows - 1] = 2.0
+    got = nncl.Sum(t, 1)
+    assert _native.last_plan().startswith(kernel + " "), _native.last_plan()
+    assert float(got[rows - 1]) == 32.0
+    assert bool((got[:rows - 1] == 120.0).all())
+    del t, got
+    torch.cuda.empty_cache()
