@@ -516,21 +516,21 @@ int launch_column_sum(hipStream_t stream, const float *X, float *Y, int outer, i
     int rows = CS_ROWS;
     if ((axis + rows - 1) / rows > 65535) rows = (axis + 65534) / 65535;
     const int chunks = (axis + rows - 1) / rows;
+    // row_sum_kernel: not for rows shorter than 16 (two lanes' worth of a tile) or fewer than
+    // 64 (lanes of every tile idle). With 512 or more work-groups of rows, or one group of
+    // chunks, a work-group takes whole rows, and there are no chunk sums to keep.
+    const int64_t blocks = ((int64_t)outer + RS_TILE - 1) / RS_TILE;
+    const bool by_row = inner == 1 && !accumulate && rows == CS_ROWS && outer >= 64 &&
+                        axis >= 16 && blocks <= kMaxGroups;
+    const bool whole = by_row && (chunks <= 4 || blocks >= 512);
     float *dst = Y;
-    if (chunks > 1) {
+    if (chunks > 1 && !whole) {
         int st = MIGEMM_OK;
         dst = static_cast<float *>(
             workspace(stream, (size_t)chunks * outer * inner * sizeof(float), &st));
         if (dst == nullptr) return st;
     }
-    const int64_t blocks = ((int64_t)outer + RS_TILE - 1) / RS_TILE;
-    if (inner == 1 && !accumulate && rows == CS_ROWS && outer >= 64 && axis >= 16 &&
-        blocks <= kMaxGroups) {
-        // Rows shorter than 16 stay below: two lanes' worth of a tile. Fewer than 64 rows
-        // would leave lanes of every tile idle.
-        // with 512 or more work-groups of rows, or one group of chunks, a work-group takes
-        // whole rows
-        const bool whole = chunks <= 4 || blocks >= 512;
+    if (by_row) {
         if (whole)
             MIGEMM_LAUNCH(row_sum_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, X,
                           Y, outer, axis);

@@ -2,6 +2,8 @@
 rows ending inside a tile of 64 columns or a chunk of 256, rows off 16-byte boundaries. The
 bits must be those of the documented order: 256 values at a time ascending from +0.0f, the
 chunk sums added in chunk order."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -53,3 +55,24 @@ def test_more_rows_than_one_launch_holds(nncl, rows, kernel):
     assert bool((got[:rows - 1] == 120.0).all())
     del t, got
     torch.cuda.empty_cache()
+
+
+def test_whole_rows_are_captured_without_a_workspace(nncl):
+    """A work-group that sums whole rows keeps no chunk sums: captured on a stream that holds
+    no workspace, replays agree with the eager sum."""
+    t = torch.randn(32768, 1283, device="cuda:0")
+    expect = nncl.Sum(t, 1)
+    cap = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        got = nncl.Sum(t, 1)
+    for _ in range(3):
+        got.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, expect)
+    size = ctypes.c_size_t(1)
+    _native.call("migemm_workspace_size", ctypes.c_void_p(cap.cuda_stream), ctypes.byref(size))
+    assert size.value == 0
