@@ -49,6 +49,13 @@ PEAK_HBM_GBS = 8000.0          # MI355X HBM3E
 # gemm_split_kernel computes each fp32 product as six bf16 products on the bf16 MFMA (2516.6
 # TFLOP/s dense), so its roofline peak in fp32 FLOP is a sixth of that rate
 PEAK_SPLIT_TFLOPS = round(2516.6 / 6, 1)
+
+
+def mfma_peak(plan):
+    """TFLOP/s of fp32 products that the matrix cores a plan runs on can reach."""
+    return PEAK_SPLIT_TFLOPS if plan.startswith("tiled-split ") else PEAK_FP32_MFMA_TFLOPS
+
+
 N4096 = 4096
 FLOP_4096 = 2.0 * N4096 ** 3
 EVENT_EVERY = 2  # timed steps per step whose launches carry HIP events
@@ -573,15 +580,16 @@ def measure_all_configs(torch, nncl, _native, calls=100):
         tf = flop / (ms * 1e-3) / 1e12
         gbs = byts / (ms * 1e-3) / 1e9
         fns[0]()
+        plan = _native.last_plan()
         out[name] = {"us": round(ms * 1e3, 2), "tflops": round(tf, 3),
-                     "pct_mfma_peak": round(100 * tf / PEAK_FP32_MFMA_TFLOPS, 2),
+                     "pct_mfma_peak": round(100 * tf / mfma_peak(plan), 2),
                      "GBps": round(gbs, 1), "pct_hbm_peak": round(100 * gbs / PEAK_HBM_GBS, 2),
                      "bound": bound,
-                     "frac": round((tf / PEAK_FP32_MFMA_TFLOPS) if bound == "mfma"
+                     "frac": round((tf / mfma_peak(plan)) if bound == "mfma"
                                    else (gbs / PEAK_HBM_GBS), 4),
                      "x_launch_floor": round(ms * 1e3 / floor_us, 2),
                      "launch_floor_us": round(floor_us, 2),
-                     "kernel": _native.last_plan()}
+                     "kernel": plan}
         if floor is not None:
             fl_ms = timed(floor[1])
             out[name]["data_floor"] = {"us": round(fl_ms * 1e3, 2), "kernel": floor[0]}
@@ -801,7 +809,7 @@ def measure_callers(torch, nncl, _native):
         e = {"us": round(ms * 1e3, 1), "kernel": _native.last_plan()}
         if flop:
             tf = flop / (ms * 1e-3) / 1e12
-            e.update(tflops=round(tf, 1), frac_mfma=round(tf / PEAK_FP32_MFMA_TFLOPS, 3))
+            e.update(tflops=round(tf, 1), frac_mfma=round(tf / mfma_peak(e["kernel"]), 3))
         if byts:
             gbs = byts / (ms * 1e-3) / 1e9
             e.update(GBps=round(gbs, 1), frac_hbm=round(gbs / PEAK_HBM_GBS, 3))

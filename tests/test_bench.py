@@ -28,12 +28,15 @@ def test_more_than_one_gpu_exits_with_a_message():
     assert "one GPU" in msg["error"]
 
 
-KERNEL = ("void migemm::(anonymous namespace)::gemm_direct_kernel<256, 256, 8, 2, {a}, {b}, 32, "
-          "2, 2, 1, 4, 4>(migemm::TiledArgs)")
+KERNELS = [("void migemm::(anonymous namespace)::gemm_direct_kernel<256, 256, 8, 2, {a}, {b}, 32, "
+            "2, 2, 1, 4, 4>(migemm::TiledArgs)"),
+           ("void migemm::(anonymous namespace)::gemm_split_kernel<256, 128, 4, 2, {a}, {b}>"
+            "(migemm::TiledArgs)")]
 FORMS = {"NN": ("true", "false"), "NT": ("true", "true"), "TN": ("false", "false")}
 
 
-def test_summarize_trace_averages_exactly_the_timed_launches(tmp_path):
+@pytest.mark.parametrize("kernel", KERNELS, ids=["direct", "split"])
+def test_summarize_trace_averages_exactly_the_timed_launches(tmp_path, kernel):
     """Each form runs once to record its plan, W warm-up times, S timed times, and may run
     again later (other configs); only the S timed launches may enter PROFILED_US."""
     steps, warmup = 4, 3
@@ -48,7 +51,7 @@ def test_summarize_trace_averages_exactly_the_timed_launches(tmp_path):
                 # shifted by one launch changes the average
                 us = 900.0 + rng.integers(0, 20) if phase == "timed" else 5000.0
                 durations[f].append((phase, us))
-                rows.append({"Kernel_Name": KERNEL.format(a=FORMS[f][0], b=FORMS[f][1]),
+                rows.append({"Kernel_Name": kernel.format(a=FORMS[f][0], b=FORMS[f][1]),
                              "Start_Timestamp": str(t), "End_Timestamp": str(t + int(us * 1e3))})
                 t += int(us * 1e3) + 5000
     # an unrelated kernel in between must not disturb the selection
@@ -85,6 +88,13 @@ def test_committed_profiles_feed_the_roofline():
         floor_us = bench.FLOP_4096 / (bench.PEAK_FP32_MFMA_TFLOPS * 1e12) * 1e6
         assert floor_us == pytest.approx(873.7, abs=0.1)
         assert floor_us <= prof[f] < 1.2 * floor_us, (f, prof[f])
+    # the bench's roofline reads those of the split kernel, which runs the forms
+    prof = bench.load_profiled(bench.SPLIT_TRACE_SUMMARY)
+    for f in FORMS:
+        traffic = bench.load_traffic(f, bench.SPLIT_PMC_SUMMARY)
+        assert traffic is not None and alg <= traffic < 4 * alg, (f, traffic)
+        floor_us = bench.FLOP_4096 / (bench.PEAK_SPLIT_TFLOPS * 1e12) * 1e6
+        assert floor_us <= prof[f] < 2.5 * floor_us, (f, prof[f])
 
 
 def test_algorithmic_work_per_config():
@@ -99,6 +109,8 @@ def test_algorithmic_work_per_config():
     assert c["3_lstm_gate_step"][:2] == (2 * M * N * K, 4 * (M * K + K * N + M * N + N))
     # the stateful form reads x_t (512) and h_{t-1} (1024) separately: the same bytes
     assert c["3h_lstm_hid_step"][:2] == c["3_lstm_gate_step"][:2]
+    assert bench.mfma_peak("tiled-split tile=128x128 splits=1") == bench.PEAK_SPLIT_TFLOPS
+    assert bench.mfma_peak("tiled-direct tile=64x64") == bench.PEAK_FP32_MFMA_TFLOPS
     assert c["5a_ragged"][:2] == (2 * 1000 * 3000 * 777,
                                   4 * (1000 * 777 + 777 * 3000 + 1000 * 3000))
     assert c["5b_gemv"][:2] == (2 * 4096 * 11008, 4 * (4096 + 4096 * 11008 + 11008))
