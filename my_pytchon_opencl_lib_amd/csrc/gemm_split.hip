@@ -49,7 +49,7 @@
 //  * Values the parts cannot carry: an infinity, a NaN or a value of 4.04e31 or more leaves
 //    its outputs not finite, and so does a sum of 4.83e24 or more. A work-group that meets one
 //    computes its tile once more with v_mfma_f32_32x32x2_f32, so these give what the fp32
-//    kernels give (such a tile costs about 2.5 times an ordinary one).
+//    kernels give (such a tile costs 2.2-2.6 times an ordinary one: 4096^3 1777, in fp32 910).
 //
 // Measured (events around 10 launches, N(0,1) operands, us, this kernel / the fp32 choice):
 // 4096^3 NN 673 / 916, NT 667 / 912, TN 692 / 916 (199-206 TFLOP/s; one sum in 256x256 tiles
